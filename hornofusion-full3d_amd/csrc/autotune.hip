@@ -6,7 +6,9 @@
 // and blocks per CU in {4, 8, 16} (capped by the tile count) or one block
 // per tile.  For the mixed solver the column-marching stencil is then timed
 // at 1 .. 16 r-segments.  The fastest shape is kept in the batch; solvers
-// pick it up at their next solve.
+// pick it up at their next solve.  Where a solver also has a resident form
+// for the batch, that is timed against the best shape and the faster of the
+// two is kept.
 #include <cfloat>
 
 #include "batch.hpp"
@@ -14,6 +16,7 @@
 namespace eafp {
 
 int time_fp64_kernels(Batch& B, int reps, float* ms_spmv, float* ms_update);
+int time_resident64(Batch& B, int iters, float* ms);
 int time_mixed_kernels(Batch& B, int fmt, int precond, int reps, float* ms_spmv, float* ms_update);
 
 // solver 0: FP64 CG; 1: mixed with the Jacobi inner preconditioner; 2:
@@ -66,6 +69,14 @@ int autotune(Batch& B, int solver, int fmt, int reps, int* best_cpt, int* best_b
             }
         }
         EAFP_TRY_RC(B.set_columns(bs));
+    }
+    // the FP64 CG with the systems on chip, where they fit: kept when it is
+    // faster than the best streaming shape
+    if (solver == 0) {
+        float ms = 0.f;
+        EAFP_TRY_RC(time_resident64(B, 16 * reps, &ms));
+        B.resident64 = ms > 0.f && ms < best;
+        if (B.resident64) best = ms;
     }
     if (best_cpt) *best_cpt = bc;
     if (best_blocks) *best_blocks = bb;

@@ -164,6 +164,8 @@ struct Batch {
     DevBuf<unsigned char> lab_bits;      // link, anchor and root bits per cell
     DevBuf<int> lab_small;               // per-system flags, root lists and counts
     long label_sweeps = 0;               // sweeps of the last labelling
+    bool resident64 = true;              // FP64 CG: on chip where the plan allows it (false: streaming kernels)
+    bool resident_mixed = true;          // mixed inner iterations: the same
     hipStream_t stream = nullptr;
     int grid = 0;                        // blocks per tile-walking launch
     Cg64Work* cg64 = nullptr;

@@ -162,12 +162,16 @@ int eafp_batch_solve_mixed(eafp_batch* b, const eafp_mixed_opts* opts, eafp_stat
 
 int eafp_batch_set_tiling(eafp_batch* b, int cells_per_thread, int blocks) {
     if (!b) return EAFP_ERR_ARG;
-    return b->B.set_tiling(cells_per_thread, blocks);
+    const int rc = b->B.set_tiling(cells_per_thread, blocks);
+    if (rc == EAFP_OK) b->B.resident64 = b->B.resident_mixed = false;   // a launch shape asked for: the kernels that have one
+    return rc;
 }
 
 int eafp_batch_set_columns(eafp_batch* b, int r_splits) {
     if (!b) return EAFP_ERR_ARG;
-    return b->B.set_columns(r_splits);
+    const int rc = b->B.set_columns(r_splits);
+    if (rc == EAFP_OK) b->B.resident64 = b->B.resident_mixed = false;
+    return rc;
 }
 
 int eafp_batch_get_columns(const eafp_batch* b, int* r_splits) {

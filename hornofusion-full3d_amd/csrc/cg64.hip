@@ -26,42 +26,13 @@
 // Algorithmic HBM bytes per cell and iteration (FP64): k64_spmv reads 7
 // coefficients + z + pv_old and writes pv_new + q (88 B); k64_update reads
 // phi, r, pv_new, q, aP and writes phi, r, z (64 B): 152 B/cell/iter.
+#include <memory>
 #include <vector>
 
-#include "batch.hpp"
+#include "cg64.hpp"
+#include "resident_plan.hpp"
 
 namespace eafp {
-
-struct CgSlot {
-    double bnorm;      // ||Su||; < 0 until the first k64_spmv after k64_init
-    double residual;   // relative recurrence residual of the last completed iteration
-    double rz, alpha, beta;
-    int it;            // iteration in progress (set by k64_spmv)
-    int n_iter;        // completed iterations
-    int done, status;
-};
-
-struct CgConst {
-    double tol;
-    int max_iter;
-    int pad;
-};
-
-struct Cg64Args {
-    const TileDesc* tiles;
-    int ntiles;
-    int nsys;
-    const double *aW, *aE, *aS, *aN, *aB, *aT, *aP;
-    const double *b, *fold, *x0;
-    double *x, *r, *z, *q;
-    double* p[2];
-    double* partA;       // ntiles:     p.q
-    double* partB;       // ntiles * 3: r.r, r.z, Su.Su
-    CgSlot* slot[2];
-    const CgConst* cst;
-    int* ndone;          // finished systems, counted after each chunk
-    int state_first;     // 1 (batches): read a system's state before its cell loads; 0: overlap them
-};
 
 struct Cg64Work {
     DevBuf<double> x, r, z, q, p0, p1, partA, partB;
@@ -74,7 +45,15 @@ struct Cg64Work {
     GraphCache<Cg64Args> graphs;    // one instantiated graph per (chunk, shape, buffers)
     hipGraphExec_t exec = nullptr;  // the cached graph of the current solve
     Cg64Args args{};
+    std::unique_ptr<ResDevice> res;  // resident solve, when the batch fits on chip
+    DevBuf<double> zx;               // its exchange buffer
+    CgSlot* slots_host = nullptr;    // pinned: the slots after a resident launch
+    unsigned* gate_host = nullptr;   // pinned: its gate word
 };
+
+ResPlan plan_resident64(const Batch& B);
+int start_resident64(Batch& B, CgSlot* slot, CgConst* cst, double tol, int max_iter);
+int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int iters);
 
 void free_cg64(Cg64Work* w) {
     if (!w) return;
@@ -84,6 +63,8 @@ void free_cg64(Cg64Work* w) {
     if (w->t0) (void)hipEventDestroy(w->t0);
     if (w->t1) (void)hipEventDestroy(w->t1);
     if (w->ndone_host) (void)hipHostFree(w->ndone_host);
+    if (w->slots_host) (void)hipHostFree(w->slots_host);
+    if (w->gate_host) (void)hipHostFree(w->gate_host);
     delete w;
 }
 
@@ -389,6 +370,15 @@ static int init_cg64(Batch& B, Cg64Work* w) {
         EAFP_TRY(hipEventCreate(&w->t1));
         EAFP_TRY(hipMemset(w->p0.p, 0, n * sizeof(double)));
         EAFP_TRY(hipMemset(w->p1.p, 0, n * sizeof(double)));
+        ResPlan plan = plan_resident64(B);
+        if (plan.ok) {
+            auto d = std::make_unique<ResDevice>();
+            EAFP_TRY_RC(w->zx.alloc(plan.xlen));
+            EAFP_TRY(hipHostMalloc((void**)&w->slots_host, sizeof(CgSlot) * B.nsys, hipHostMallocDefault));
+            EAFP_TRY(hipHostMalloc((void**)&w->gate_host, sizeof(unsigned), hipHostMallocDefault));
+            EAFP_TRY_RC(d->init(std::move(plan), B.stream));
+            w->res = std::move(d);
+        }
     }
     return EAFP_OK;
 }
@@ -486,11 +476,67 @@ static int cg64_graph(Batch& B, int chunk) {
     return EAFP_OK;
 }
 
+static int fill_stats(const Batch& B, const CgSlot* st, eafp_stats* stats) {
+    float ms = 0.f;
+    EAFP_TRY(hipEventElapsedTime(&ms, B.cg64->t0, B.cg64->t1));
+    if (!stats) return EAFP_OK;
+    for (int s = 0; s < B.nsys; ++s) {
+        eafp_stats& o = stats[s];
+        o = eafp_stats{};
+        o.residual = st[s].residual;
+        o.n_iter = st[s].n_iter;
+        o.n_refine = 0;
+        o.status = st[s].status;
+        o.true_rel_l2 = -1.0;
+        o.true_rel_l1 = -1.0;
+        o.seconds = ms * 1e-3;
+    }
+    return EAFP_OK;
+}
+
+// The solve with the systems on chip: one launch per RES_ITERS iterations of
+// every system (a launch leaves the state of unfinished systems in the
+// streaming kernels' arrays and the next one takes it up; about 0.3 % of an
+// iteration's time at 1024, and no launch runs for long).  *done = 0
+// when the launch was given up (resident.hpp): nothing is written that the
+// streaming kernels read.
+constexpr int RES_ITERS = 1024;
+static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* stats, int* done) {
+    Cg64Work* w = B.cg64;
+    ResDevice& D = *w->res;
+    *done = 0;
+    EAFP_TRY(hipEventRecord(w->t0, B.stream));
+    EAFP_TRY_RC(start_resident64(B, w->slot1.p, w->cst.p, tol, max_iter));
+    const ResidentGate held(D.plan.T > 1 ? D.plan.nteam * D.plan.T : 0);
+    for (;;) {
+        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, RES_ITERS));
+        for (int s = 0; s < B.nsys; ++s) EAFP_TRY_RC(download_x(B, s, w->x.p));
+        EAFP_TRY(hipEventRecord(w->t1, B.stream));
+        EAFP_TRY(hipMemcpyAsync(w->slots_host, w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));
+        EAFP_TRY(hipMemcpyAsync(w->gate_host, D.gate.p, sizeof(unsigned), hipMemcpyDeviceToHost, B.stream));
+        EAFP_TRY(hipStreamSynchronize(B.stream));
+        if (*w->gate_host & GATE_GIVEN_UP) {
+            D.given_up = true;
+            return EAFP_OK;
+        }
+        bool all = true;
+        for (int s = 0; s < B.nsys; ++s) all = all && w->slots_host[s].done;
+        if (all) break;
+    }
+    *done = 1;
+    return fill_stats(B, w->slots_host, stats);
+}
+
 int solve_fp64(Batch& B, int max_iter, double tol, eafp_stats* stats, int chunk) {
     for (int s = 0; s < B.nsys; ++s)
         if (!B.uploaded[s]) return EAFP_ERR_STATE;
     EAFP_TRY_RC(ensure_cg64(B));
     Cg64Work* w = B.cg64;
+    if (B.resident64 && w->res && !w->res->given_up) {
+        int done = 0;
+        EAFP_TRY_RC(solve_fp64_resident(B, max_iter, tol, stats, &done));
+        if (done) return EAFP_OK;
+    }
     if (chunk <= 0) chunk = 16;
     chunk = (chunk + 1) & ~1;    // even: the pv buffer parity restarts every chunk
     EAFP_TRY_RC(cg64_graph(B, chunk));
@@ -536,21 +582,38 @@ int solve_fp64(Batch& B, int max_iter, double tol, eafp_stats* stats, int chunk)
     std::vector<CgSlot> st(B.nsys);
     EAFP_TRY(hipMemcpyAsync(st.data(), w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));
     EAFP_TRY(hipStreamSynchronize(B.stream));
-    float ms = 0.f;
-    EAFP_TRY(hipEventElapsedTime(&ms, w->t0, w->t1));
-    if (stats) {
-        for (int s = 0; s < B.nsys; ++s) {
-            eafp_stats& o = stats[s];
-            o = eafp_stats{};
-            o.residual = st[s].residual;
-            o.n_iter = st[s].n_iter;
-            o.n_refine = 0;
-            o.status = st[s].status;
-            o.true_rel_l2 = -1.0;
-            o.true_rel_l1 = -1.0;
-            o.seconds = ms * 1e-3;
-        }
+    return fill_stats(B, st.data(), stats);
+}
+
+// One iteration of every system on chip (ms), over about `iters` of them
+// (tol = 0), the launch's own loads and stores included; 0 when the batch has
+// no resident form.
+int time_resident64(Batch& B, int iters, float* ms) {
+    *ms = 0.f;
+    for (int s = 0; s < B.nsys; ++s)
+        if (!B.uploaded[s]) return EAFP_ERR_STATE;
+    EAFP_TRY_RC(ensure_cg64(B));
+    Cg64Work* w = B.cg64;
+    if (!w->res || w->res->given_up) return EAFP_OK;
+    ResDevice& D = *w->res;
+    const ResidentGate held(D.plan.T > 1 ? D.plan.nteam * D.plan.T : 0);
+    for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
+        EAFP_TRY_RC(start_resident64(B, w->slot1.p, w->cst.p, 0.0, 1 << 30));
+        EAFP_TRY(hipEventRecord(w->t0, B.stream));
+        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, iters));
+        EAFP_TRY(hipEventRecord(w->t1, B.stream));
+        EAFP_TRY(hipMemcpyAsync(w->slots_host, w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));
+        EAFP_TRY(hipMemcpyAsync(w->gate_host, D.gate.p, sizeof(unsigned), hipMemcpyDeviceToHost, B.stream));
+        EAFP_TRY(hipStreamSynchronize(B.stream));
     }
+    if (*w->gate_host & GATE_GIVEN_UP) {
+        D.given_up = true;
+        return EAFP_OK;
+    }
+    int n = 1;
+    for (int s = 0; s < B.nsys; ++s) n = std::max(n, w->slots_host[s].n_iter);
+    EAFP_TRY(hipEventElapsedTime(ms, w->t0, w->t1));
+    *ms /= (float)n;
     return EAFP_OK;
 }
 

@@ -1,0 +1,70 @@
+// resident_plan.hpp -- host side of the resident solvers: which batches
+// they take, the teams, and the launch's device tables.
+#pragma once
+#include <vector>
+
+#include "batch.hpp"
+#include "resident.hpp"
+
+namespace eafp {
+
+// What a resident kernel of one solver can hold and about what its
+// iterations cost; the plan picks the team size by it.
+struct ResLimits {
+    int max_slots;                            // slots per thread
+    int (*slots)(int nz, int rows);           // slots per thread for `rows` z-rows, 0: none fits
+    size_t (*lds)(int nz, int rows, int lds_rows, int halo_rows);
+    float sync_us[9];                         // two team sums and the exchange, T = 1, 2, 4 .. 256
+    float slot_us;                            // one slot's iteration
+};
+
+struct ResPlan {
+    bool ok = false;
+    int nsys = 0;
+    int T = 0, nteam = 0, blocks = 0;
+    int slots = 0;                            // largest over the items
+    size_t lds = 0;
+    int max_items = 0;                        // longest team list
+    float est_us = 0.f;                       // model: one iteration of every system
+    std::vector<ResItem> items;               // team by team
+    std::vector<int> team_begin;
+    long xlen = 0;                            // elements of the exchange buffer
+};
+
+// The plan for a batch, or !ok when a system fits no team.  `xpitch`: the
+// exchange buffer's elements per z-row.
+ResPlan plan_resident(const std::vector<SysGeom>& g, const ResLimits& lim, int (*xpitch)(int nz));
+
+// Work-groups of resident launches in flight on this process's GPUs: a launch
+// takes its number before it is queued and gives it back when it has ended,
+// waiting in turn when the CUs are taken, so that two launches never hold
+// half of the CUs each.
+class ResidentGate {
+  public:
+    explicit ResidentGate(int blocks);
+    ~ResidentGate();
+    ResidentGate(const ResidentGate&) = delete;
+    ResidentGate& operator=(const ResidentGate&) = delete;
+
+  private:
+    int dev_, n_;
+};
+
+// A plan's tables on the device.
+struct ResDevice {
+    ResPlan plan;
+    DevBuf<ResItem> items;
+    DevBuf<int> team_begin;
+    DevBuf<u64> slots;
+    DevBuf<unsigned> gate;
+    unsigned tag = 1;             // first tag of the next launch
+    bool given_up = false;        // a launch did not get its CUs: stream from now on
+    int init(ResPlan&& p, hipStream_t stream);
+    ResLaunch launch() const;
+    // gate open and `tag` set for the next launch, which uses at most `tags` of them
+    int arm(long tags, hipStream_t stream);
+};
+
+__global__ void k_res_arm(unsigned* gate, unsigned tag);
+
+}  // namespace eafp

@@ -318,7 +318,10 @@ int eafp_batch_info(const eafp_batch* b, int* grid, int* tile_cells, long* ncell
 
 /* Launch shape of every kernel of the batch: a tile of 256*cells_per_thread
  * cells (cells_per_thread in {1, 2, 4, 8}) and `blocks` blocks per launch
- * (0: one per tile, at most 8 per CU).  No reference counterpart. */
+ * (0: one per tile, at most 8 per CU).  From this call on the solves of the
+ * batch use the kernels that have such a shape, instead of keeping systems
+ * on chip where they fit (the default), until eafp_batch_autotune decides
+ * anew; so does eafp_batch_set_columns.  No reference counterpart. */
 int eafp_batch_set_tiling(eafp_batch* b, int cells_per_thread, int blocks);
 
 /* The mixed solver's stencil as a column march: r_splits > 0 cuts every
@@ -348,7 +351,9 @@ int eafp_batch_time_kernels(eafp_batch* b, int solver, int coef_format, int reps
  * the solver's iteration kernels (solver as for eafp_batch_time_kernels)
  * and keeps the fastest; for the mixed solver it then times the
  * column-marching stencil at 1, 2, 4, 6, 8, 10, 12 and 16 r-segments and
- * keeps it if it is faster (eafp_batch_get_columns tells).
+ * keeps it if it is faster (eafp_batch_get_columns tells); where the solver
+ * can keep the systems on chip, that is timed too and used if it is faster
+ * still.
  * Returns the tile shape and the iteration time (ms).  No reference
  * counterpart. */
 int eafp_batch_autotune(eafp_batch* b, int solver, int coef_format, int reps, int* cells_per_thread,

@@ -1,0 +1,93 @@
+"""The resident solvers (systems kept on chip) on the GPU, at the sizes where
+their division of a system changes form: one cell per axis, an uncut and a cut
+theta ring, rows longer than a work-group, one member and many, the largest
+number of cells per thread, and solves that a second launch takes up.
+
+Default batches take the resident form; a launch shape asked for
+(set_tiling) takes the streaming kernels.  Iterates after a few iterations
+differ between the two only by the order of the sums, a few units of the
+last place each: 1e-12 of the largest value, as the oracle comparison of
+tests/test_gpu_cg64.py has it.
+"""
+import numpy as np
+import pytest
+
+import eafp
+import oracle
+from eafp import systems
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1, 1), (1, 1, 5), (1, 3, 700), (3, 1, 7), (2, 2, 1), (5, 2, 33), (7, 50, 20), (9, 8, 64), (33, 17, 65),
+          (40, 64, 3), (18, 36, 24), (35, 66, 50), (60, 119, 83)]
+
+
+def system(shape, index=0):
+    if min(shape[0], shape[1], shape[2]) > 4:
+        return systems.make_system(2, index, shape)
+    # the generator's masks leave no cell on the thinnest meshes: a random
+    # diagonally dominant system instead
+    rng = np.random.default_rng([index, *shape])
+    g = systems.make_geometry(*shape)
+    ps = systems.assemble(g, np.ones(shape, dtype=bool), np.full(shape, 1.2), tuple(rng.uniform(0.5, 2.0, shape)
+                                                                                   for _ in range(3)), rng)
+    ps.coef["aP"][2:-2, 2:-2, 2:-2] += rng.uniform(0.01, 0.1, shape) * ps.coef["aP"][2:-2, 2:-2, 2:-2].max()
+    ps.Su[2:-2, 2:-2, 2:-2] = rng.normal(size=shape)
+    return ps
+
+
+def both(syss, solve):
+    out = []
+    for stream in (False, True):
+        with eafp.Batch.from_systems(syss) as b:
+            if stream:
+                b.set_tiling(2, 0)
+            st = solve(b)
+            out.append((st, [b.download(s) for s in range(len(syss))]))
+    return out
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("max_iter", [0, 1, 2, 9])
+def test_fp64_iterates(shape, max_iter):
+    ps = system(shape)
+    (st, phi), (st_s, phi_s) = both([ps], lambda b: b.solve_fp64(max_iter, 1e-30))
+    ref, _, nit, _ = oracle.cg(ps, max_iter=max_iter, tol=1e-30)
+    print(f"case fp64 {shape} {max_iter}: {st[0]['status']} {st_s[0]['status']} n {st[0]['n_iter']} {nit}", flush=True)
+    assert st[0]["status"] == st_s[0]["status"] and st[0]["n_iter"] == st_s[0]["n_iter"] == nit
+    scale = max(np.abs(ref).max(), 1e-300)
+    assert np.abs(phi[0] - phi_s[0]).max() <= 1e-12 * scale
+    assert np.abs(oracle.interior(phi[0]) - oracle.interior(ref)).max() <= 1e-12 * scale
+
+
+def test_fp64_past_one_launch():
+    """1306 iterations to 1e-8: the second launch goes on where the first one
+    stopped."""
+    ps = systems.make_system(2)
+    (st, phi), (st_s, phi_s) = both([ps], lambda b: b.solve_fp64(tol=1e-8))
+    assert st[0]["status"] == "converged" and st[0]["n_iter"] > 1024
+    assert abs(st[0]["n_iter"] - st_s[0]["n_iter"]) <= 2
+    assert oracle.gauge_error(oracle.interior(phi[0]), oracle.interior(phi_s[0]), ps.labels, ps.ncomp) < 1e-9
+
+
+def test_fp64_uneven_batch_with_failures():
+    """Teams with several systems each; a zero right-hand side, a NaN and a
+    thin mesh among them; repeats are bit-identical."""
+    syss = [systems.make_system(3, s) for s in range(20)] + [system((1, 3, 700))]
+    zero, nan = systems.make_system(1, 1), systems.make_system(1, 2)
+    zero.Su[:] = 0.0
+    nan.Su[6, 7, 8] = np.nan
+    syss += [zero, nan]
+    with eafp.Batch.from_systems(syss) as b:
+        st = b.solve_fp64(1500, 1e-8)
+        phi = [b.download(s) for s in range(len(syss))]
+        again = b.solve_fp64(1500, 1e-8)
+        for s in range(len(syss)):
+            np.testing.assert_array_equal(b.download(s), phi[s])
+            assert again[s]["n_iter"] == st[s]["n_iter"]
+    assert st[-2]["status"] == "zero_rhs" and st[-2]["n_iter"] == 0
+    assert st[-1]["status"] == "max_iter" and st[-1]["n_iter"] == 1500 and np.isnan(st[-1]["residual"])
+    for s in (0, 7, 19):
+        ref, _, nit, _ = oracle.cg(syss[s])
+        assert st[s]["status"] == "converged" and abs(st[s]["n_iter"] - nit) <= 2
+        assert oracle.gauge_error(oracle.interior(phi[s]), oracle.interior(ref), syss[s].labels, syss[s].ncomp) < 1e-9
