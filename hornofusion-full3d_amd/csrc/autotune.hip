@@ -17,6 +17,7 @@ namespace eafp {
 
 int time_fp64_kernels(Batch& B, int reps, float* ms_spmv, float* ms_update);
 int time_resident64(Batch& B, int iters, float* ms);
+int time_resident_mixed(Batch& B, int fmt, int precond, int iters, float* ms);
 int time_mixed_kernels(Batch& B, int fmt, int precond, int reps, float* ms_spmv, float* ms_update);
 
 // solver 0: FP64 CG; 1: mixed with the Jacobi inner preconditioner; 2:
@@ -69,9 +70,13 @@ int autotune(Batch& B, int solver, int fmt, int reps, int* best_cpt, int* best_b
             }
         }
         EAFP_TRY_RC(B.set_columns(bs));
+        float ms = 0.f;
+        EAFP_TRY_RC(time_resident_mixed(B, fmt, solver == 2 ? EAFP_PRECOND_ZLINE : EAFP_PRECOND_JACOBI, 32, &ms));
+        B.resident_mixed = ms > 0.f && ms < best;
+        if (B.resident_mixed) best = ms;
     }
-    // the FP64 CG with the systems on chip, where they fit: kept when it is
-    // faster than the best streaming shape
+    // the systems on chip, where they fit: kept when that is faster than the
+    // best streaming shape
     if (solver == 0) {
         float ms = 0.f;
         EAFP_TRY_RC(time_resident64(B, 16 * reps, &ms));

@@ -164,15 +164,18 @@ __global__ __launch_bounds__(RB, 2) void k64_resident(R64Args g) {
         };
         // the neighbours' edge rows, into Zh
         auto fetch = [&](int w, int n) {
-            wait_members(t, S, mem);
             constexpr int Q = U >= R64_TIGHT ? 4 : 8;
-            for (int h0 = w * 64 + (tid & 63); h0 < nhalo; h0 += Q * 64 * n) {
-                double v[Q];
+            for (int h0 = w * 64 + (tid & 63), first = 1; first || h0 < nhalo; h0 += Q * 64 * n, first = 0) {
+                int src[Q];
 #pragma unroll
                 for (int q = 0; q < Q; ++q) {
                     const int h = h0 + q * 64 * n;
-                    v[q] = ld_agent_d(zx + H[h < nhalo ? h : h0].x);
+                    src[q] = h < nhalo ? H[h].x : 0;
                 }
+                if (first) wait_members(t, S, mem);
+                double v[Q];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) v[q] = ld_agent_d(zx + src[q]);
 #pragma unroll
                 for (int q = 0; q < Q; ++q)
                     if (h0 + q * 64 * n < nhalo) Zh[h0 + q * 64 * n] = v[q];
@@ -267,6 +270,8 @@ __global__ __launch_bounds__(RB, 2) void k64_resident(R64Args g) {
                 const double pc = P[lo[u]];
                 z[u] = (flag[u] & F_CELL) ? apply(u, pc) : 0.0;   // q, until z is formed again
                 acc1[0] += pc * z[u];
+                formed(z[u]);
+                formed(acc1[0]);
             }
             alive = team_sum<1>(t, acc1, S, false, NoAside());
             if (!alive) break;
@@ -289,6 +294,11 @@ __global__ __launch_bounds__(RB, 2) void k64_resident(R64Args g) {
                 z[u] = ok ? zz : 0.0;
                 acc[0] += r[u] * r[u];
                 acc[1] += r[u] * z[u];
+                formed(x(u));
+                formed(r[u]);
+                formed(z[u]);
+                formed(acc[0]);
+                formed(acc[1]);
             }
             publish();
             alive = team_sum<2>(t, acc, S, true, fetch);

@@ -36,132 +36,13 @@
 // One captured graph runs a whole refinement step for every system:
 // interval x (k_mspmv, k_mupdate), k_res, k_rsum, k_mreplace, k_mcount.
 #include <cmath>
+#include <memory>
 #include <vector>
 
-#include "batch.hpp"
+#include "mixed.hpp"
+#include "mixed_resident.hpp"
 
 namespace eafp {
-
-// Per-system state of the mixed solver, double-buffered by kernel role:
-// MxDyn changes every inner iteration (k_mspmv reads slot 1 and writes
-// slot 0, k_mupdate the reverse); MxStat changes once per refinement step
-// (k_res copies slot 1 to slot 0, k_mreplace writes slot 1 from slot 0).
-// Every thread loads the few MxDyn fields it needs and the writer stores
-// its new values straight from registers.
-struct MxDyn {
-    double rz, alpha, beta;
-    int fresh;          // next k_mspmv starts a new Krylov sequence (beta = 0)
-    int broken;         // inner breakdown: idle until the next refinement step
-    int total_inner;
-    int done;           // mirror of MxStat::done for the inner kernels
-};
-
-struct MxStat {
-    double bnorm, b1, res_l2, res_l1;
-    double mean_x[MAX_COMP];
-    int n_refine, done, status, xbuf;
-};
-
-struct MxConst {
-    double tol;
-    double inv_cnt[MAX_COMP];
-    int ncomp, max_steps, restart, pad;
-};
-
-constexpr int NRES = 4 + 2 * MAX_COMP;   // r.r, |r|, Su.Su, |Su|, sum r per comp, sum x per comp
-
-struct MxArgs {
-    const TileDesc* tiles;
-    int ntiles;
-    int nsys;
-    const ColDesc* cols;   // column segments (column-marching stencil)
-    // FP64 operand
-    const double *aW, *aE, *aS, *aN, *aB, *aT, *aP, *b, *fold, *x0;
-    const unsigned char* comp;
-    double* X[2];        // FP64 iterate, ping-pong per refinement step
-    double* r64;         // FP64 residual of the current refinement step
-    double* xout;        // projected result
-    // compressed operand
-    void* w[3];          // +r, +theta, +z face weights (format dependent)
-    float* scale;        // FP16 only: per-cell scale (the owner's aP)
-    void* e;             // diagonal excess, in the weight format (FP16: scaled like the weights)
-    float* dinv;         // Jacobi inverse of the rounded operator
-    const LineTile* lt;  // line tiles (z-line preconditioner)
-    unsigned* fac;       // z-line factors per cell: FP16 l (low half), BF16 1/d (high half)
-    int line;            // 1: z-line preconditioner; the r.z partials are per line tile
-    int state_first;     // 1 (batches): read the system's state before the cell loads, so the
-                         // blocks of converged systems load nothing; 0 (one system): overlap them
-    // inner FP32 vectors
-    float *d, *r, *z, *q;
-    float* p[2];
-    long sink;           // a 16-byte slot past the cells of p[0], p[1] and q: stores that must be issued but not kept
-    double* partR;       // ntiles * NRES (k_res)
-    double* sumR;        // nsys * NRES: partR reduced per system (k_rsum)
-    const SysGeom* geom; // per-system geometry and tile ranges
-    double* partA;       // ntiles        (k_mspmv: p.q)
-    double* partB;       // ntiles * 2, or nltiles * 2 with `line` (k_mreplace, k_mupdate: r.r, r.z)
-    MxDyn* dyn[2];
-    MxStat* stat[2];
-    const MxConst* cst;
-    int* ndone;
-};
-
-// ---------------------------------------------------------------------------
-// Weight storage formats
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ unsigned short f32_to_bf16_rne(float v) {
-    unsigned u = __float_as_uint(v);
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
-
-template <int F>
-struct WFmt;
-
-template <>
-struct WFmt<EAFP_COEF_FP32> {
-    using T = float;
-    __device__ static float load(const void* w, const float*, long o) { return ((const float*)w)[o]; }
-    __device__ static F4 load4(const void* w, const float*, long o) { return ld4((const float*)w + o); }
-    __device__ static T enc(float v, float) { return v; }
-    __device__ static float dec(T h, float) { return h; }
-};
-
-template <>
-struct WFmt<EAFP_COEF_BF16> {
-    using T = unsigned short;
-    __device__ static float load(const void* w, const float*, long o) {
-        return __uint_as_float((unsigned)((const unsigned short*)w)[o] << 16);
-    }
-    __device__ static F4 load4(const void* w, const float*, long o) {
-        unsigned short h[4];
-        __builtin_memcpy(h, __builtin_assume_aligned((const unsigned short*)w + o, 8), 8);
-        F4 r;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) r.v[q] = __uint_as_float((unsigned)h[q] << 16);
-        return r;
-    }
-    __device__ static T enc(float v, float) { return f32_to_bf16_rne(v); }
-    __device__ static float dec(T h, float) { return __uint_as_float((unsigned)h << 16); }
-};
-
-template <>
-struct WFmt<EAFP_COEF_FP16> {
-    using T = _Float16;
-    __device__ static float load(const void* w, const float* sc, long o) {
-        return (float)((const _Float16*)w)[o] * sc[o];
-    }
-    __device__ static F4 load4(const void* w, const float* sc, long o) {
-        _Float16 h[4];
-        __builtin_memcpy(h, __builtin_assume_aligned((const _Float16*)w + o, 8), 8);
-        F4 r = ld4(sc + o);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) r.v[q] *= (float)h[q];
-        return r;
-    }
-    __device__ static T enc(float v, float s) { return (_Float16)(v / s); }
-    __device__ static float dec(T h, float s) { return (float)h * s; }
-};
 
 size_t wbytes(int fmt) { return fmt == EAFP_COEF_FP32 ? 4 : 2; }
 
@@ -1337,15 +1218,6 @@ __device__ __forceinline__ unsigned pack_fac(double l, double inv) {
     return (unsigned)lb | ((unsigned)f32_to_bf16_rne((float)inv) << 16);
 }
 
-__device__ __forceinline__ void unpack_fac(float bits, float& l, float& inv) {
-    const unsigned u = __float_as_uint(bits);
-    const unsigned short lb = (unsigned short)(u & 0xFFFFu);
-    _Float16 lh;
-    __builtin_memcpy(&lh, &lb, 2);
-    l = (float)lh;
-    inv = __uint_as_float(u & 0xFFFF0000u);
-}
-
 // One thread per line, k = 0 .. nz-1 in order (once per solve, after
 // k_compress has left D in q).
 template <int F>
@@ -1761,12 +1633,25 @@ __global__ __launch_bounds__(BLOCK) void k_mreplace_line(MxArgs a) {
     store_run<2>(a.partB, (int)blockIdx.x, 1, 1, acc);
 }
 
-__global__ __launch_bounds__(BLOCK) void k_mcount(MxArgs a) {
+// Finished systems; -1 when a resident launch was given up.  Opens the gate
+// of the next resident launch, whose tags begin after this one's.
+__global__ __launch_bounds__(BLOCK) void k_mcount(MxArgs a, unsigned* gate, unsigned tags) {
     __shared__ double sh[BLOCK / 64];
     double v[1] = {0.0};
     for (int s = threadIdx.x; s < a.nsys; s += BLOCK) v[0] += a.stat[1][s].done ? 1.0 : 0.0;
     block_sum<1>(v, sh);
-    if (threadIdx.x == 0) *a.ndone = (int)v[0];
+    if (threadIdx.x == 0) {
+        int n = (int)v[0];
+        if (gate) {
+            if (gate[0] & GATE_GIVEN_UP) {
+                n = -1;
+            } else {
+                gate[0] = 0;
+                gate[1] += tags;
+            }
+        }
+        *a.ndone = n;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1798,8 +1683,6 @@ __global__ __launch_bounds__(BLOCK) void k_mproject(MxArgs a, int tile) {
     }
 }
 
-constexpr long SINK_CELLS = 64;   // past the arenas of p and q: the column stencil's discarded stores
-
 struct MixedWork {
     int fmt = -1;
     DevBuf<double> X0, X1, r64, xout, partR, partA, partB, sumR;
@@ -1817,6 +1700,9 @@ struct MixedWork {
     GraphCache<MxArgs> graphs;      // one instantiated graph per (format, interval, precond, shape, buffers)
     hipGraphExec_t exec = nullptr;  // the cached graph of the current solve
     MxArgs args{};
+    std::unique_ptr<ResDevice> res; // resident inner iterations, when the batch fits on chip
+    int res_cq = 1;                 // quads per lane
+    DevBuf<float> xz;               // their exchange buffer
 };
 
 void free_mixed(MixedWork* w) {
@@ -1832,6 +1718,38 @@ void free_mixed(MixedWork* w) {
 
 int download_x(Batch& B, int s, const double* x_compact);
 
+// Slots (rows per wave and lane) and LDS of a resident work-group with CQ
+// quads per lane.
+template <int CQ>
+static int rmx_slots(int nz, int rows) {
+    const int nl = rmx_lanes(nz, CQ);
+    if (nl > 64) return 0;
+    return (rows + RW * (64 / nl) - 1) / (RW * (64 / nl));
+}
+template <int CQ>
+static size_t rmx_lds(int nz, int, int lds_rows, int halo_rows) {
+    return rmx_scratch() + ((size_t)(lds_rows + halo_rows) * 16 + (size_t)halo_rows * 8) * rmx_lanes(nz, CQ) * CQ;
+}
+template <int CQ>
+static int rmx_pitch(int nz) {
+    return rmx_lanes(nz, CQ) * CQ * 4;
+}
+
+// The mixed batch's resident plan, with one or two quads per lane, whichever
+// the model gives the shorter iteration (not ok: the batch streams).
+static ResPlan plan_resident_mixed(const Batch& B, int* cq) {
+    // fitted to BF16 z-line iterations: 8.6 us (T 256, 2 slots of one quad), 8.7
+    // (128, 3), 10.8 (64, 5), 15.5 (32, 10), 10.0 (16, 5), 14.6 (8, 10); with two
+    // quads 10.6 (64, 3), 12.4 (8, 5)
+    static const ResLimits lim1 = {10, rmx_slots<1>, rmx_lds<1>,
+                                   {1.2f, 4.5f, 4.5f, 5.0f, 5.0f, 5.8f, 5.6f, 5.6f, 6.2f}, 0.95f};
+    static const ResLimits lim2 = {5, rmx_slots<2>, rmx_lds<2>,
+                                   {1.2f, 4.5f, 4.5f, 5.0f, 5.0f, 5.8f, 5.6f, 5.6f, 6.2f}, 1.9f};
+    ResPlan p1 = plan_resident(B.geom, lim1, rmx_pitch<1>), p2 = plan_resident(B.geom, lim2, rmx_pitch<2>);
+    *cq = p2.ok && (!p1.ok || p2.est_us < p1.est_us) ? 2 : 1;
+    return *cq == 2 ? std::move(p2) : std::move(p1);
+}
+
 // First-time buffers of the mixed solver; the caller publishes w only when
 // every one of them exists.
 static int init_mixed(Batch& B, MixedWork* w) {
@@ -1841,7 +1759,7 @@ static int init_mixed(Batch& B, MixedWork* w) {
         EAFP_TRY_RC(w->X1.alloc(n));
         EAFP_TRY_RC(w->r64.alloc(n));
         EAFP_TRY_RC(w->xout.alloc(n));
-        EAFP_TRY_RC(w->dinv.alloc(n));
+        EAFP_TRY_RC(w->dinv.alloc(n + SINK_CELLS));
         EAFP_TRY_RC(w->d.alloc(n));
         EAFP_TRY_RC(w->r.alloc(n));
         EAFP_TRY_RC(w->z.alloc(n));
@@ -1849,6 +1767,7 @@ static int init_mixed(Batch& B, MixedWork* w) {
         EAFP_TRY_RC(w->p0.alloc(n + SINK_CELLS));
         EAFP_TRY_RC(w->p1.alloc(n + SINK_CELLS));
         EAFP_TRY(hipMemset(w->d.p, 0, n * sizeof(float)));
+        EAFP_TRY(hipMemset(w->dinv.p, 0, (n + SINK_CELLS) * sizeof(float)));
         EAFP_TRY(hipMemset(w->p0.p, 0, (n + SINK_CELLS) * sizeof(float)));
         EAFP_TRY(hipMemset(w->p1.p, 0, (n + SINK_CELLS) * sizeof(float)));
         EAFP_TRY_RC(w->dyn0.alloc(B.nsys));
@@ -1861,6 +1780,13 @@ static int init_mixed(Batch& B, MixedWork* w) {
         for (auto& e : w->ev) EAFP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         EAFP_TRY(hipEventCreate(&w->t0));
         EAFP_TRY(hipEventCreate(&w->t1));
+        ResPlan plan = plan_resident_mixed(B, &w->res_cq);
+        if (plan.ok) {
+            auto d = std::make_unique<ResDevice>();
+            EAFP_TRY_RC(w->xz.alloc(plan.xlen));
+            EAFP_TRY_RC(d->init(std::move(plan), B.stream));
+            w->res = std::move(d);
+        }
     }
     return EAFP_OK;
 }
@@ -1879,16 +1805,29 @@ static int ensure_mixed(Batch& B, int fmt) {
     if (w->fmt != fmt) {
         const size_t n = B.ncells;
         w->fmt = -1;   // a failed allocation below leaves the weights invalid, not stale
-        for (auto& wb : w->w) EAFP_TRY_RC(wb.alloc(n * wbytes(fmt)));
-        EAFP_TRY_RC(w->e.alloc(n * wbytes(fmt)));
-        if (fmt == EAFP_COEF_FP16) EAFP_TRY_RC(w->scale.alloc(n));
+        // the cells between and past the systems are read (the rest of a
+        // quad that begins at a row's last cell), so they hold numbers
+        const size_t nb = (n + SINK_CELLS) * wbytes(fmt);
+        for (auto& wb : w->w) {
+            EAFP_TRY_RC(wb.alloc(nb));
+            EAFP_TRY(hipMemsetAsync(wb.p, 0, nb, B.stream));
+        }
+        EAFP_TRY_RC(w->e.alloc(nb));
+        EAFP_TRY(hipMemsetAsync(w->e.p, 0, nb, B.stream));
+        if (fmt == EAFP_COEF_FP16) {
+            EAFP_TRY_RC(w->scale.alloc(n + SINK_CELLS));
+            EAFP_TRY(hipMemsetAsync(w->scale.p, 0, (n + SINK_CELLS) * sizeof(float), B.stream));
+        }
         w->fmt = fmt;
     }
     EAFP_TRY_RC(w->partR.alloc((size_t)B.ntiles * NRES));
     EAFP_TRY_RC(w->sumR.alloc((size_t)B.nsys * NRES));
     EAFP_TRY_RC(w->partA.alloc((size_t)B.ntiles));
     EAFP_TRY_RC(w->partB.alloc((size_t)std::max(B.ntiles, B.nltiles) * 2));
-    if (B.nltiles > 0 && !w->fac.p) EAFP_TRY_RC(w->fac.alloc(B.ncells));
+    if (B.nltiles > 0 && !w->fac.p) {
+        EAFP_TRY_RC(w->fac.alloc(B.ncells + SINK_CELLS));
+        EAFP_TRY(hipMemsetAsync(w->fac.p, 0, (B.ncells + SINK_CELLS) * sizeof(unsigned), B.stream));
+    }
     MxArgs& a = w->args;
     a.tiles = B.tiles.p;
     a.ntiles = B.ntiles;
@@ -2000,26 +1939,62 @@ static void launch_refine(Batch& B) {
     else k_mreplace<<<B.grid, BLOCK, 0, B.stream>>>(B.mixed->args, tile);
 }
 
+static int rmx_prepare(int fmt, bool line, int cq, int slots) {
+    if (fmt == EAFP_COEF_BF16) return rmx_prepare_bf16(line, cq, slots);
+    if (fmt == EAFP_COEF_FP16) return rmx_prepare_fp16(line, cq, slots);
+    return rmx_prepare_fp32(line, cq, slots);
+}
+
+// Tags that one resident launch of `interval` inner iterations uses at most.
+static long resident_tags(const ResDevice& D, int interval) { return D.plan.max_items * (2L * interval + 2); }
+
+// The inner iterations of one refinement step, on chip.
+static int launch_resident_mixed(Batch& B, int fmt, int interval) {
+    MixedWork* w = B.mixed;
+    const ResPlan& p = w->res->plan;
+    RMxArgs g{};
+    g.a = w->args;
+    g.L = w->res->launch();
+    g.xz = w->xz.p;
+    g.interval = interval;
+    const size_t lds = std::max(p.lds, p.T > 1 ? (size_t)RES_LDS_ALONE : (size_t)0);
+    const bool line = w->args.line != 0;
+    if (fmt == EAFP_COEF_BF16) return rmx_launch_bf16(line, w->res_cq, p.slots, g, p.blocks, lds, B.stream);
+    if (fmt == EAFP_COEF_FP16) return rmx_launch_fp16(line, w->res_cq, p.slots, g, p.blocks, lds, B.stream);
+    return rmx_launch_fp32(line, w->res_cq, p.slots, g, p.blocks, lds, B.stream);
+}
+
 // The graph of one refinement step for every system.  Looked up in the
 // workspace's cache by format, interval, preconditioner, launch shape and
 // every buffer its kernels name; captured and instantiated on a miss.
-static int mixed_graph(Batch& B, int fmt, int interval) {
+static int mixed_graph(Batch& B, int fmt, int interval, bool resident) {
     MixedWork* w = B.mixed;
-    const int key[GraphCache<MxArgs>::kKeys] = {fmt, interval, w->args.line, 0};
+    const int key[GraphCache<MxArgs>::kKeys] = {fmt, interval, w->args.line, resident ? 1 : 0};
     w->exec = w->graphs.find(key, B.tiling_gen, w->args);
     if (w->exec) return EAFP_OK;
     EAFP_TRY(hipStreamSynchronize(B.stream));   // no earlier launch of a graph that make_room may drop
     w->graphs.make_room(B.tiling_gen);
     hipGraph_t graph = nullptr;
+    if (resident) EAFP_TRY_RC(rmx_prepare(fmt, w->args.line != 0, w->res_cq, w->res->plan.slots));
     EAFP_TRY(hipStreamBeginCapture(B.stream, hipStreamCaptureModeThreadLocal));
-    for (int c = 0; c < interval; ++c) {
-        launch_mspmv(B, fmt, c & 1);
-        launch_mupdate(B, c & 1);
+    int rc = EAFP_OK;
+    if (resident) {
+        rc = launch_resident_mixed(B, fmt, interval);
+    } else {
+        for (int c = 0; c < interval; ++c) {
+            launch_mspmv(B, fmt, c & 1);
+            launch_mupdate(B, c & 1);
+        }
     }
     launch_refine(B);
-    k_mcount<<<1, BLOCK, 0, B.stream>>>(w->args);
+    k_mcount<<<1, BLOCK, 0, B.stream>>>(w->args, resident ? w->res->gate.p : nullptr,
+                                        resident ? (unsigned)resident_tags(*w->res, interval) : 0u);
     hipError_t e = hipStreamEndCapture(B.stream, &graph);
     if (e != hipSuccess) return (int)e;
+    if (rc != EAFP_OK) {
+        (void)hipGraphDestroy(graph);
+        return rc;
+    }
     hipGraphExec_t exec = nullptr;
     e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
@@ -2078,21 +2053,21 @@ static int check_mixed(Batch& B, const eafp_mixed_opts& o) {
     return EAFP_OK;
 }
 
-int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
-    EAFP_TRY_RC(check_mixed(B, o));
-    const int fmt = o.coef_format;
-    EAFP_TRY_RC(ensure_mixed(B, fmt));
+// Setup and the refinement steps until every system is finished.  *given_up:
+// a resident launch did not get its CUs (resident.hpp), the solve has to
+// begin again.  Returns with the stream idle but for the launch after the
+// last one needed.
+static int mixed_steps(Batch& B, const eafp_mixed_opts& o, int fmt, int interval, bool resident, int* given_up) {
     MixedWork* w = B.mixed;
-    w->args.line = o.precond == EAFP_PRECOND_ZLINE ? 1 : 0;
-    int interval = o.interval > 0 ? o.interval : 32;
-    interval = (interval + 1) & ~1;    // even: the p buffer parity restarts every step
-    EAFP_TRY_RC(mixed_graph(B, fmt, interval));
-    EAFP_TRY(hipEventRecord(w->t0, B.stream));
+    *given_up = 0;
+    EAFP_TRY_RC(mixed_graph(B, fmt, interval, resident));
+    const long max_launch = (long)o.max_steps + 2;
+    const long tags = resident ? resident_tags(*w->res, interval) : 0;
+    if (resident) EAFP_TRY_RC(w->res->arm(0, B.stream));
     EAFP_TRY_RC(mixed_start(B, o, fmt));
 
     // One graph launch = one refinement step for every system; poll the
     // finished count of the step before the one just launched.
-    const long max_launch = (long)o.max_steps + 2;
     long launched = 0;
     for (;;) {
         if (launched < max_launch) {
@@ -2102,17 +2077,53 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
             EAFP_TRY(hipMemcpyAsync(&w->host_cnt[slot], w->ndone.p, sizeof(int), hipMemcpyDeviceToHost, B.stream));
             EAFP_TRY(hipEventRecord(w->ev[slot], B.stream));
             ++launched;
+            if (resident) w->res->tag += (unsigned)tags;
+            if (resident && w->res->tag > 0xF0000000u - 2 * (unsigned)tags) {   // begin the tags again
+                EAFP_TRY(hipStreamSynchronize(B.stream));
+                if (w->host_cnt[slot] < 0) {
+                    *given_up = 1;
+                    return EAFP_OK;
+                }
+                EAFP_TRY_RC(w->res->arm(0x20000000, B.stream));
+                w->res->tag = 1;
+            }
         }
         if (launched >= 2) {
             const int older = (int)(launched & 1);
             EAFP_TRY(hipEventSynchronize(w->ev[older]));
-            if (w->host_cnt[older] >= B.nsys) break;
+            if (w->host_cnt[older] >= B.nsys || w->host_cnt[older] < 0) break;
         }
         if (launched >= max_launch) {
             EAFP_TRY(hipEventSynchronize(w->ev[(launched - 1) & 1]));
             break;
         }
     }
+    if (resident) {
+        EAFP_TRY(hipStreamSynchronize(B.stream));   // the CUs are free again
+        *given_up = w->host_cnt[(launched - 1) & 1] < 0;
+    }
+    return EAFP_OK;
+}
+
+int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
+    EAFP_TRY_RC(check_mixed(B, o));
+    const int fmt = o.coef_format;
+    EAFP_TRY_RC(ensure_mixed(B, fmt));
+    MixedWork* w = B.mixed;
+    w->args.line = o.precond == EAFP_PRECOND_ZLINE ? 1 : 0;
+    int interval = o.interval > 0 ? o.interval : 32;
+    interval = (interval + 1) & ~1;    // even: the p buffer parity restarts every step
+    EAFP_TRY(hipEventRecord(w->t0, B.stream));
+    int given_up = 0;
+    if (B.resident_mixed && w->res && !w->res->given_up) {
+        const ResPlan& p = w->res->plan;
+        const ResidentGate held(p.T > 1 ? p.nteam * p.T : 0);
+        EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, true, &given_up));
+        w->res->given_up = given_up != 0;
+    } else {
+        given_up = 1;
+    }
+    if (given_up) EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, false, &given_up));
     k_mproject<<<B.grid, BLOCK, 0, B.stream>>>(w->args, BLOCK * B.cpt);
     EAFP_TRY(hipGetLastError());
     for (int s = 0; s < B.nsys; ++s) EAFP_TRY_RC(download_x(B, s, w->xout.p));
@@ -2137,6 +2148,43 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
             out.seconds = ms * 1e-3;
         }
     }
+    return EAFP_OK;
+}
+
+// One inner iteration of every system on chip (ms), over `iters` of them, the
+// launch's own loads and stores included; 0 when the batch has no resident
+// form.
+int time_resident_mixed(Batch& B, int fmt, int precond, int iters, float* ms) {
+    *ms = 0.f;
+    eafp_mixed_opts o{};
+    o.tol = 1e-300;
+    o.max_steps = 1 << 20;
+    o.coef_format = fmt;
+    o.precond = precond;
+    EAFP_TRY_RC(check_mixed(B, o));
+    EAFP_TRY_RC(ensure_mixed(B, fmt));
+    MixedWork* w = B.mixed;
+    if (!w->res || w->res->given_up) return EAFP_OK;
+    w->args.line = precond == EAFP_PRECOND_ZLINE ? 1 : 0;
+    ResDevice& D = *w->res;
+    EAFP_TRY_RC(rmx_prepare(fmt, w->args.line != 0, w->res_cq, D.plan.slots));
+    const ResidentGate held(D.plan.T > 1 ? D.plan.nteam * D.plan.T : 0);
+    for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
+        EAFP_TRY_RC(mixed_start(B, o, fmt));
+        EAFP_TRY_RC(D.arm(resident_tags(D, iters), B.stream));
+        EAFP_TRY(hipEventRecord(w->t0, B.stream));
+        EAFP_TRY_RC(launch_resident_mixed(B, fmt, iters));
+        EAFP_TRY(hipEventRecord(w->t1, B.stream));
+        k_mcount<<<1, BLOCK, 0, B.stream>>>(w->args, D.gate.p, 0u);
+        EAFP_TRY(hipMemcpyAsync(&w->host_cnt[0], w->ndone.p, sizeof(int), hipMemcpyDeviceToHost, B.stream));
+        EAFP_TRY(hipStreamSynchronize(B.stream));
+    }
+    if (w->host_cnt[0] < 0) {
+        D.given_up = true;
+        return EAFP_OK;
+    }
+    EAFP_TRY(hipEventElapsedTime(ms, w->t0, w->t1));
+    *ms /= (float)iters;
     return EAFP_OK;
 }
 

@@ -366,6 +366,12 @@ __device__ __forceinline__ int fresh(int v) {
     return v;
 }
 
+// The value is formed by here: what leads to it is not put off past this
+// point (to after a whole loop over the thread's cells, say, with everything
+// it needs kept in registers meanwhile).
+__device__ __forceinline__ void formed(float& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void formed(double& v) { asm volatile("" : "+v"(v)); }
+
 // A value that is the same in every lane, in scalar registers.
 template <typename R>
 __device__ __forceinline__ R uniform(const R& v) {

@@ -91,3 +91,83 @@ def test_fp64_uneven_batch_with_failures():
         ref, _, nit, _ = oracle.cg(syss[s])
         assert st[s]["status"] == "converged" and abs(st[s]["n_iter"] - nit) <= 2
         assert oracle.gauge_error(oracle.interior(phi[s]), oracle.interior(ref), syss[s].labels, syss[s].ncomp) < 1e-9
+
+
+# z-rows: one cell to one more than a wave holds with one quad per lane, and
+# with two; the last one streams
+ROWS = [(5, 7, 1), (4, 6, 3), (6, 5, 4), (3, 9, 63), (4, 6, 64), (5, 4, 65), (16, 24, 84), (4, 5, 129), (3, 8, 168),
+        (3, 4, 255), (2, 3, 257), (2, 3, 512), (2, 2, 513)]
+BIG = [(18, 36, 24), (35, 66, 49), (60, 120, 84), (61, 119, 83)]
+
+
+def true_residual(ps, phi):
+    l2, _ = oracle.true_residual(ps, phi)
+    return l2
+
+
+@pytest.mark.parametrize("shape", ROWS + BIG)
+@pytest.mark.parametrize("precond", [eafp._lib.PRECOND_JACOBI, eafp._lib.PRECOND_ZLINE])
+@pytest.mark.parametrize("fmt", [eafp._lib.COEF_FP32, eafp._lib.COEF_BF16, eafp._lib.COEF_FP16])
+def test_mixed_matches_streaming(shape, precond, fmt):
+    """Both forms end the same way.  Where they reach the tolerance, they do
+    so on the caller's FP64 operator and with the same solution.  (The inner
+    counts are not compared: the streaming forms' own differ by up to two
+    refinement steps with the order of their sums.  On meshes that the inner CG solves in
+    fewer iterations than a refinement step has, the kept search direction
+    can stall the refinement with rounded weights, in both forms alike.)"""
+    ps = system(shape, 3)
+    c0 = eafp.counters()["graph_launches"]
+    (st, phi), (st_s, phi_s) = both([ps], lambda b: b.solve_mixed(tol=1e-9, coef_format=fmt, precond=precond))
+    launches = eafp.counters()["graph_launches"] - c0
+    print(f"case mixed {shape} fmt {fmt} precond {precond}: inner {st[0]['n_iter']} {st_s[0]['n_iter']}", flush=True)
+    assert st[0]["status"] == st_s[0]["status"]
+    if st[0]["status"] != "converged":
+        assert min(shape) < 18 and 0.1 < st[0]["residual"] / st_s[0]["residual"] < 10.0
+        return
+    for s, x in ((st[0], phi[0]), (st_s[0], phi_s[0])):
+        assert s["residual"] < 1e-9
+        assert true_residual(ps, x) < 1.2e-9
+    assert launches <= st[0]["n_refine"] + st_s[0]["n_refine"] + 4    # no launch was given up and solved again
+    assert oracle.gauge_error(oracle.interior(phi[0]), oracle.interior(phi_s[0]), ps.labels, ps.ncomp) < 1e-6
+
+
+@pytest.mark.parametrize("precond", [eafp._lib.PRECOND_JACOBI, eafp._lib.PRECOND_ZLINE])
+def test_mixed_uneven_batch_with_failures(precond):
+    """Teams with several systems each; a zero right-hand side and a NaN among
+    them; restart mode; repeats are bit-identical."""
+    syss = [systems.make_system(3, s) for s in range(40)] + [system((6, 5, 4))]
+    zero, nan = systems.make_system(1, 1), systems.make_system(1, 2)
+    zero.Su[:] = 0.0
+    nan.Su[6, 7, 8] = np.nan
+    syss += [zero, nan]
+    for restart in (False, True):
+        with eafp.Batch.from_systems(syss) as b:
+            st = b.solve_mixed(tol=1e-8, max_steps=60, coef_format=eafp._lib.COEF_BF16, precond=precond, restart=restart)
+            phi = [b.download(s) for s in range(len(syss))]
+            again = b.solve_mixed(tol=1e-8, max_steps=60, coef_format=eafp._lib.COEF_BF16, precond=precond,
+                                  restart=restart)
+            for s in range(len(syss)):
+                np.testing.assert_array_equal(b.download(s), phi[s])
+                assert again[s]["n_iter"] == st[s]["n_iter"]
+            b.set_tiling(2, 0)
+            streamed = b.solve_mixed(tol=1e-8, max_steps=60, coef_format=eafp._lib.COEF_BF16, precond=precond,
+                                     restart=restart)
+        print(f"case mixed batch precond {precond} restart {restart}: {[x['status'] for x in st]}", flush=True)
+        assert [x["status"] for x in st] == [x["status"] for x in streamed]
+        assert st[-2]["status"] == "zero_rhs"
+        assert st[-1]["status"] == "max_iter" and np.isnan(st[-1]["residual"])
+        for s in range(41):
+            if st[s]["status"] == "converged":
+                assert true_residual(syss[s], phi[s]) < 1.2e-8
+
+
+def test_fp64_default_does_not_stream():
+    """A default FP64 solve launches no graph of the streaming kernels."""
+    ps = systems.make_system(1)
+    c0 = eafp.counters()["graph_launches"]
+    with eafp.Batch.from_systems([ps]) as b:
+        b.solve_fp64(tol=1e-8)
+        assert eafp.counters()["graph_launches"] == c0
+        b.set_tiling(2, 0)
+        b.solve_fp64(tol=1e-8)
+        assert eafp.counters()["graph_launches"] > c0
