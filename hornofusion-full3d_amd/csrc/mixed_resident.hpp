@@ -80,6 +80,16 @@ struct WQuad<EAFP_COEF_FP16> {
     __device__ __forceinline__ float get(int k) const { return (float)h[k] * s.v[k]; }
 };
 
+// a where bit `n` of f is set, else b: a sign-extended bit and a bitwise
+// select (a compare and a conditional move wait for each other, 17 cycles
+// against 9).
+template <int BIT>
+__device__ __forceinline__ int pick(unsigned f, int a, int b) {
+    constexpr int n = __builtin_ctz(BIT);
+    const int m = (int)(f << (31 - n)) >> 31;
+    return (a & m) | (b & ~m);
+}
+
 // The six weight pieces of a lane's quads, loaded one slot ahead of their use.
 template <int F, int CQ>
 struct WSet {
@@ -88,15 +98,10 @@ struct WSet {
 
 // Lane shifts over the whole wave; the end lane gets 0.
 __device__ __forceinline__ float from_prev_lane(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xF, 0xF, false));   // wave_shr:1
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138, 0xF, 0xF, true));   // wave_shr:1
 }
 __device__ __forceinline__ float from_next_lane(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xF, 0xF, false));   // wave_shl:1
-}
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float old, float v) {
-    return __int_as_float(
-        __builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, 0xF, 0xF, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130, 0xF, 0xF, true));   // wave_shl:1
 }
 __device__ __forceinline__ float readlane_f(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
@@ -104,36 +109,59 @@ __device__ __forceinline__ float readlane_f(float v, int l) {
 
 // The value that flows into each lane: lane n's map y -> A y + B applied to
 // what flows into it flows into lane n+1 (UP) or n-1; 0 flows into the end.
+// Steps of 1, 2, 4, 8 lanes inside the rows of 16, two instructions each (a
+// lane without a source adds 0 to B and keeps A); then the row ends.  The
+// shifted operand is part of the multiply: as moves of their own, each step
+// took 40 cycles of the wave instead of 12.  A shifted operand needs two
+// wait states after its write, which the other chain and the s_nop make.
 template <bool UP>
 __device__ __forceinline__ float scan_lanes(float A, float B) {
-    const int lane = threadIdx.x & 63;
-#define EAFP_SCAN_STEP(S)                                            \
-    {                                                                \
-        const float Ap = dpp_f<(UP ? 0x110 : 0x100) + S>(1.f, A);    \
-        const float Bp = dpp_f<(UP ? 0x110 : 0x100) + S>(0.f, B);    \
-        B = A * Bp + B;                                              \
-        A = A * Ap;                                                  \
-    }
-    EAFP_SCAN_STEP(1)
-    EAFP_SCAN_STEP(2)
-    EAFP_SCAN_STEP(4)
-    EAFP_SCAN_STEP(8)
-#undef EAFP_SCAN_STEP
-    // what flows into each row of 16 lanes
-    float x;
     if (UP) {
-        const float x1 = readlane_f(B, 15);
-        const float x2 = readlane_f(A, 31) * x1 + readlane_f(B, 31);
-        const float x3 = readlane_f(A, 47) * x2 + readlane_f(B, 47);
-        x = lane < 16 ? 0.f : lane < 32 ? x1 : lane < 48 ? x2 : x3;
-    } else {
-        const float x2 = readlane_f(B, 48);
-        const float x1 = readlane_f(A, 32) * x2 + readlane_f(B, 32);
-        const float x0 = readlane_f(A, 16) * x1 + readlane_f(B, 16);
-        x = lane < 16 ? x0 : lane < 32 ? x1 : lane < 48 ? x2 : 0.f;
+        asm("s_nop 1\n\t"
+            "v_fmac_f32_dpp %1, %1, %0 row_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+            "v_mul_f32_dpp %0, %0, %0 row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_fmac_f32_dpp %1, %1, %0 row_shr:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+            "v_mul_f32_dpp %0, %0, %0 row_shr:2 row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_fmac_f32_dpp %1, %1, %0 row_shr:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+            "v_mul_f32_dpp %0, %0, %0 row_shr:4 row_mask:0xf bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_fmac_f32_dpp %1, %1, %0 row_shr:8 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+            "v_mul_f32_dpp %0, %0, %0 row_shr:8 row_mask:0xf bank_mask:0xf\n\t"
+            // the end of rows 0 and 2 into rows 1 and 3, then of row 1 into rows 2 and 3
+            "s_nop 0\n\t"
+            "v_fmac_f32_dpp %1, %1, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "v_mul_f32_dpp %0, %0, %0 row_bcast:15 row_mask:0xa bank_mask:0xf\n\t"
+            "s_nop 0\n\t"
+            "v_fmac_f32_dpp %1, %1, %0 row_bcast:31 row_mask:0xc bank_mask:0xf"
+            : "+v"(A), "+v"(B));
+        return from_prev_lane(B);
     }
-    const float y = A * x + B;                         // what flows out of each lane
-    return dpp_f<(UP ? 0x111 : 0x101)>(x, y);
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %1, %1, %0 row_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_mul_f32_dpp %0, %0, %0 row_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0\n\t"
+        "v_fmac_f32_dpp %1, %1, %0 row_shl:2 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_mul_f32_dpp %0, %0, %0 row_shl:2 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0\n\t"
+        "v_fmac_f32_dpp %1, %1, %0 row_shl:4 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_mul_f32_dpp %0, %0, %0 row_shl:4 row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 0\n\t"
+        "v_fmac_f32_dpp %1, %1, %0 row_shl:8 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+        "v_mul_f32_dpp %0, %0, %0 row_shl:8 row_mask:0xf bank_mask:0xf"
+        : "+v"(A), "+v"(B));
+    // what flows out of the first lanes of rows 3, 2 and 1 flows into rows 2, 1 and 0
+    const float x2 = readlane_f(B, 48);
+    const float x1 = readlane_f(A, 32) * x2 + readlane_f(B, 32);
+    const float x0 = readlane_f(A, 16) * x1 + readlane_f(B, 16);
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %1, %2 quad_perm:[0,1,2,3] row_mask:0x4 bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %3 quad_perm:[0,1,2,3] row_mask:0x2 bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %4 quad_perm:[0,1,2,3] row_mask:0x1 bank_mask:0xf"
+        : "+v"(B)
+        : "v"(A), "v"(x2), "v"(x1), "v"(x0));
+    return from_next_lane(B);
 }
 
 // z = M^-1 r for the wave's rows: L y = r upwards, L^T z = y/d downwards.
@@ -227,7 +255,7 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
         const int k0 = j * NC;
         // rows in order: wave by wave, slot by slot
         float r[U][NC], d[U][NC], q[U][NC];
-        int lo[U], gr[U];                          // first quad in LDS; row in the system
+        int lo[U], go[U];                          // first quad in LDS; first cell in the system, or the pad's
         unsigned flag[U];
         enum { F_CELL = 1, F_EDGE = 2, F_W = 4, F_S = 8, F_N = 16, F_J0 = 32 };
 
@@ -244,11 +272,11 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
             const int gi = R.i0 + li, gj = R.j0 + lj;
             const bool edge = (li == 0 && R.i0 > 0) || (li == X.bi - 1 && R.i1 < I.nr) ||
                               (X.hs && (lj == 0 || lj == X.bj - 1));
-            flag[u] = (ok ? F_CELL : 0) | (ok && edge ? F_EDGE : 0) | (gi > 0 ? F_W : 0) |
-                      (!X.hs && lj == 0 ? F_S : 0) | (!X.hs && lj == X.bj - 1 ? F_N : 0) | (gj == 0 ? F_J0 : 0);
+            flag[u] = (ok ? F_CELL : 0) | (ok && edge ? F_EDGE : 0) | (gi > 0 || !ok ? F_W : 0) |
+                      (!X.hs && lj == 0 ? F_S : 0) | (!X.hs && lj == X.bj - 1 ? F_N : 0) | (ok && gj == 0 ? F_J0 : 0);
             lo[u] = X.lds_row(li, lj) * nq + j * CQ;
-            gr[u] = gi * I.nth + gj;
-            const long o = I.off + gr[u] * nz + k0;
+            go[u] = ok ? (gi * I.nth + gj) * nz + k0 : (int)pad;
+            const long o = I.off + go[u];
 #pragma unroll
             for (int k = 0; k < NC; ++k) {
                 const bool c = ok && k0 + k < nz;
@@ -280,7 +308,8 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
             for (int u = 0; u < U; ++u) {
                 const int f = fresh((int)flag[u]);
                 if (f & F_EDGE) {
-                    const int gq = fresh(gr[u]) * nq + j * CQ;
+                    const int o = fresh(go[u]);
+                    const int gq = whole ? o >> 2 : (o - k0) / nz * nq + j * CQ;
 #pragma unroll
                     for (int c = 0; c < CQ; ++c) {
                         res_u4 v;
@@ -315,13 +344,13 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
                 }
             }
         };
-        // A slot without a row reads zeros: its q and z come out 0.  Beyond the
-        // inner wall stands the outer wall's row of w_r, whose weights are 0.
+        const int eW = (int)span * (I.nr - 1), eS = (int)span - nz;
+        // A slot without a row stands at the pad, inside the arena for its W and
+        // S weights too; its q is cleared and its z comes out 0.  Beyond the inner
+        // wall stands the outer wall's row of w_r, whose weights are 0.
         auto load_w = [&](int u, WSet<F, CQ>& w) {
-            const int f = fresh((int)flag[u]);
-            const unsigned o = (f & F_CELL) ? (unsigned)(fresh(gr[u]) * nz + k0) : pad;
-            const unsigned oW = (f & F_CELL) ? ((f & F_W) ? o - span : o + span * (unsigned)(I.nr - 1)) : pad;
-            const unsigned oS = (f & F_CELL) ? ((f & F_J0) ? o + (span - (unsigned)nz) : o - (unsigned)nz) : pad;
+            const unsigned f = (unsigned)fresh((int)flag[u]), o = (unsigned)fresh(go[u]);
+            const unsigned oW = o + (unsigned)pick<F_W>(f, -(int)span, eW), oS = o + (unsigned)pick<F_J0>(f, eS, -nz);
 #pragma unroll
             for (int c = 0; c < CQ; ++c) {
                 w.wr[c].load(w0, sc, o + 4 * c);
@@ -333,7 +362,7 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
             }
         };
         auto load_pre = [&](int u, F4 (&v)[CQ]) {
-            const unsigned o = (fresh((int)flag[u]) & F_CELL) ? (unsigned)(fresh(gr[u]) * nz + k0) : pad;
+            const unsigned o = (unsigned)fresh(go[u]);
 #pragma unroll
             for (int c = 0; c < CQ; ++c) __builtin_memcpy(&v[c], pre + o + 4 * c, 16);
         };
@@ -357,21 +386,31 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
             const float fb = (float)D.beta;
             WSet<F, CQ> w;
             if (AHEAD) load_w(0, w);
-            // p = z + beta p, own rows and halo rows (each quad by one thread)
+            // p = z + beta p, own rows and halo rows (each quad by one thread);
+            // read several slots ahead of the writes
+            constexpr int PG = U * CQ <= 6 ? U : 5;
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (flag[u] & F_CELL) {
-                    float4* p = P + fresh(lo[u]);
+            for (int u0 = 0; u0 < U; u0 += PG) {
+                float4 v[PG][CQ];
+#pragma unroll
+                for (int u = u0; u < u0 + PG && u < U; ++u)
+#pragma unroll
+                    for (int c = 0; c < CQ; ++c) v[u - u0][c] = P[fresh(lo[u]) + c];
+#pragma unroll
+                for (int u = u0; u < u0 + PG && u < U; ++u) {
 #pragma unroll
                     for (int c = 0; c < CQ; ++c) {
-                        float4 v = p[c];
-                        v.x = q[u][4 * c] + fb * v.x;
-                        v.y = q[u][4 * c + 1] + fb * v.y;
-                        v.z = q[u][4 * c + 2] + fb * v.z;
-                        v.w = q[u][4 * c + 3] + fb * v.w;
-                        p[c] = v;
+                        float4& x = v[u - u0][c];
+                        x.x = q[u][4 * c] + fb * x.x;
+                        x.y = q[u][4 * c + 1] + fb * x.y;
+                        x.z = q[u][4 * c + 2] + fb * x.z;
+                        x.w = q[u][4 * c + 3] + fb * x.w;
                     }
+                    if (flag[u] & F_CELL)
+#pragma unroll
+                        for (int c = 0; c < CQ; ++c) P[lo[u] + c] = v[u - u0][c];
                 }
+            }
             for (int h = tid; h < nhalo; h += RB) {
                 float4* p = P + H[h].y;
                 const float4 z = Zh[h];
@@ -390,9 +429,9 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
                 WSet<F, CQ> wn;
                 if (AHEAD && u + 1 < U) load_w(u + 1 < U ? u + 1 : 0, wn);
                 if (!AHEAD) load_w(u, w);
-                const int f = fresh((int)flag[u]);
+                const unsigned f = (unsigned)fresh((int)flag[u]);
                 const float4* p = P + fresh(lo[u]);
-                const int lS = (f & F_S) ? wrap : -nq, lN = (f & F_N) ? -wrap : nq;
+                const int lS = pick<F_S>(f, wrap, -nq), lN = pick<F_N>(f, -wrap, nq);
                 float pc[NC], y[NC], wz[NC];
 #pragma unroll
                 for (int c = 0; c < CQ; ++c) {
@@ -420,13 +459,14 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
                     y[k] += wz[k] * (pc[k] - (k + 1 < NC ? pc[k + 1 < NC ? k + 1 : 0] : pT));
                     y[k] += (k > 0 ? wz[k > 0 ? k - 1 : 0] : wB) * (pc[k] - (k > 0 ? pc[k > 0 ? k - 1 : 0] : pB));
                 }
+                const int live = pick<F_CELL>(f, -1, 0);
                 if (!whole)
 #pragma unroll
                     for (int k = 0; k < NC; ++k) y[k] = k0 + k < nz ? y[k] : 0.f;
 #pragma unroll
                 for (int k = 0; k < NC; ++k) {
-                    q[u][k] = y[k];
-                    acc[0] += (double)pc[k] * (double)y[k];
+                    q[u][k] = __int_as_float(__float_as_int(y[k]) & live);
+                    acc[0] += (double)pc[k] * (double)q[u][k];
                     formed(q[u][k]);
                 }
                 formed(acc[0]);
@@ -490,7 +530,7 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (!(flag[u] & F_CELL)) continue;
-            const long o = I.off + gr[u] * nz + k0;
+            const long o = I.off + go[u];
 #pragma unroll
             for (int k = 0; k < NC; ++k)
                 if (k0 + k < nz) {
