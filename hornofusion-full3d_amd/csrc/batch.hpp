@@ -127,6 +127,15 @@ struct CompInfo {
 enum { CTR_UPLOADS = 0, CTR_LABELLED, CTR_CAPTURES, CTR_LAUNCHES, CTR_COUNT };
 void counter_add(int which, long long v);
 
+// One system of the download launch (batch.hip, k_phi_out).
+struct PhiOut {
+    int nr, nth, nz;
+    int tr, tz;          // tiles in r and z
+    long block0;         // its first block
+    long off;            // first cell of the system in the arenas
+    double* phi;         // its padded phi
+};
+
 struct Cg64Work;     // cg64.hip
 struct MixedWork;    // mixed.hip
 
@@ -158,6 +167,8 @@ struct Batch {
     DevBuf<unsigned char> comp;          // projected-component slot per cell (NO_COMP: none)
     std::vector<CompInfo> comp_info;
     std::vector<DevBuf<double>*> phi_pad;  // padded phi per system (device)
+    DevBuf<PhiOut> phi_out;              // the download launch's systems
+    long phi_blocks = 0;
     std::vector<char> uploaded;          // 0: no; 1: yes; 2: yes, singular components labelled
     DevBuf<double> staging;              // padded staging for uploads
     DevBuf<int> lab;                     // component labelling: a cell index per cell

@@ -68,7 +68,7 @@ void free_cg64(Cg64Work* w) {
     delete w;
 }
 
-int download_x(Batch& B, int s, const double* x_compact);
+int download_all(Batch& B, const double* x_compact);
 
 // ---------------------------------------------------------------------------
 // r = Su - A*phi0, z = r/max(|aP|,SMALL), pv_old = 0, partials r.r, r.z,
@@ -510,7 +510,7 @@ static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* s
     const ResidentGate held(D.plan.T > 1 ? D.plan.nteam * D.plan.T : 0);
     for (;;) {
         EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, RES_ITERS));
-        for (int s = 0; s < B.nsys; ++s) EAFP_TRY_RC(download_x(B, s, w->x.p));
+        EAFP_TRY_RC(download_all(B, w->x.p));
         EAFP_TRY(hipEventRecord(w->t1, B.stream));
         EAFP_TRY(hipMemcpyAsync(w->slots_host, w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));
         EAFP_TRY(hipMemcpyAsync(w->gate_host, D.gate.p, sizeof(unsigned), hipMemcpyDeviceToHost, B.stream));
@@ -577,7 +577,7 @@ int solve_fp64(Batch& B, int max_iter, double tol, eafp_stats* stats, int chunk)
             break;
         }
     }
-    for (int s = 0; s < B.nsys; ++s) EAFP_TRY_RC(download_x(B, s, w->x.p));
+    EAFP_TRY_RC(download_all(B, w->x.p));
     EAFP_TRY(hipEventRecord(w->t1, B.stream));
     std::vector<CgSlot> st(B.nsys);
     EAFP_TRY(hipMemcpyAsync(st.data(), w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));

@@ -1716,7 +1716,7 @@ void free_mixed(MixedWork* w) {
     delete w;
 }
 
-int download_x(Batch& B, int s, const double* x_compact);
+int download_all(Batch& B, const double* x_compact);
 
 // Slots (rows per wave and lane) and LDS of a resident work-group with CQ
 // quads per lane.
@@ -2126,7 +2126,7 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
     if (given_up) EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, false, &given_up));
     k_mproject<<<B.grid, BLOCK, 0, B.stream>>>(w->args, BLOCK * B.cpt);
     EAFP_TRY(hipGetLastError());
-    for (int s = 0; s < B.nsys; ++s) EAFP_TRY_RC(download_x(B, s, w->xout.p));
+    EAFP_TRY_RC(download_all(B, w->xout.p));
     EAFP_TRY(hipEventRecord(w->t1, B.stream));
     std::vector<MxStat> st(B.nsys);
     std::vector<MxDyn> dy(B.nsys);
