@@ -5,7 +5,8 @@
 // src/mod_boundary_3d.f90:180-277), for one serial mesh.
 //
 // Layout: the caller's padded Fortran arrays (bounds (-1:n+2), r fastest);
-// one thread per padded cell, halo cells write zeros.  Two kernels:
+// one thread per padded cell, halo cells write zeros.  Three kernels:
+//   k_pp_act       one byte per cell: fluid, liquid active, gas active
 //   k_pp_grad      cell pressure gradients gr, gth, gz of the liquid and gz
 //                  of the gas (whose vertical faces drop the liquid weight);
 //                  the theta halos of the gradients are read through the
@@ -21,10 +22,23 @@
 // same double the oracle restatement computes.  The continuity residual's
 // two global sums are reduced in block order on the host.
 //
-// Algorithmic bytes per padded cell: the two gradient passes read p,
-// cell_type and the activity inputs of the cell and its 6 neighbours
-// (cached), write 4 gradients (32 B); the assembly reads ~26 input arrays
-// (~200 B) and the gradients of 7 cells, writes 8 coefficient arrays (64 B).
+// Algorithmic bytes per padded cell: the activity pass reads 32 B and writes
+// 1; the gradient pass reads p, alpha_l, rho_l, T_l and the activity byte of
+// the cell and its 6 neighbours (cached), writes 4 gradients (32 B); the
+// assembly reads ~26 input arrays (~200 B) and the gradients of 7 cells,
+// writes 8 coefficient arrays (64 B).
+//
+// What bounds them is memory latency: a cell needs about a hundred values of
+// itself and its neighbours.  So every load of a phase is issued before the
+// first face is formed, and a closed face is discarded by a select: with the
+// loads inside the branches a wave went through one memory round trip per
+// face and phase, and with the activity worked out at every neighbour from
+// its six arrays it issued 36 loads more per cell.  The three kernels took 80
+// us at 61x61x63 and 119 us at 60x120x84 cells, against 94 and 127 for two
+// kernels that did so.  Holding the loads of a phase costs 204 registers (two
+// waves per SIMD); bounded to three waves the assembly spills and takes 104 us
+// against 78 on average of the two sizes, and with the phases on two threads
+// of a cell (152 registers) 110 us.
 #include <algorithm>
 #include <cmath>
 #include <mutex>
@@ -61,6 +75,7 @@ struct PPArgs {
     double dt, rho_gas, T_amb, beta;
     int two_phase, compress;
     double *gr, *gth, *gz, *gzg;
+    unsigned char* act;      // ACT_* per cell
     double *aW, *aE, *aS, *aN, *aB, *aT, *aP, *Su;
     double* part;            // 2 per block: flux_ref, sum|Su|
     int chunk;               // blocks per XCD run (cell_of_thread)
@@ -68,25 +83,9 @@ struct PPArgs {
     int* lk[3];
 };
 
-template <class A>
-__device__ __forceinline__ bool act_l(const A& a, long o) {
-    return a.liq_cont ? a.liq_cont[o] != 0 : a.al[o] >= ALPHA_FLOW_CUTOFF;
-}
-
-template <class A>
-__device__ __forceinline__ bool act_g(const A& a, long o) {
-    bool g = a.ag[o] >= ALPHA_FLOW_CUTOFF;
-    if (a.pv_active) g = g && a.pv_active[o] != 0;
-    if (a.gas_reach) g = g || (a.gas_reach[o] != 0 && a.ag[o] < ALPHA_FLOW_CUTOFF && a.ct[o] != 0);
-    return g;
-}
-
-template <class A>
-__device__ __forceinline__ bool pv_cell(const A& a, long o) { return a.ct[o] != 0 && (act_l(a, o) || act_g(a, o)); }
-
-// Cell o's fluid flag and both activity flags, the same logic as above with
-// every load issued up front (no short-circuit between loads), so the loads
-// of several cells overlap instead of forming a chain.
+// Cell o's fluid flag and both activity flags (src/mod_pressure_3d.f90:127-169),
+// with every load issued up front (no short-circuit between loads), so the
+// loads of several cells overlap instead of forming a chain.
 struct CellAct {
     bool fluid, l, g;
 };
@@ -110,6 +109,11 @@ __device__ __forceinline__ CellAct cell_act(const A& a, long o) {
 
 __device__ __forceinline__ bool pv_of(const CellAct& c) { return c.fluid && (c.l || c.g); }
 
+// The same flags of every cell as one byte (k_pp_act).
+constexpr unsigned ACT_FLUID = 1, ACT_L = 2, ACT_G = 4;
+
+__device__ __forceinline__ bool pv_of(unsigned f) { return (f & ACT_FLUID) && (f & (ACT_L | ACT_G)); }
+
 __device__ __forceinline__ double pgrad(double pm, double p0, double pp_, double xm, double x0, double xp, bool okm,
                                         bool okp) {
     if (okm && okp) return (pp_ - pm) / (xp - xm);
@@ -118,11 +122,13 @@ __device__ __forceinline__ double pgrad(double pm, double p0, double pp_, double
     return 0.0;
 }
 
-// Liquid weight on the z-face between cells a and b (src/mod_pressure_3d.f90:406-417).
-__device__ __forceinline__ double liq_weight(const PPArgs& x, long a, long b) {
-    return 0.5 * GRAVITY *
-           ((act_l(x, a) ? 1.0 : 0.0) * x.al[a] * x.rhol[a] * (1.0 - x.beta * (x.Tl[a] - x.T_amb)) +
-            (act_l(x, b) ? 1.0 : 0.0) * x.al[b] * x.rhol[b] * (1.0 - x.beta * (x.Tl[b] - x.T_amb)));
+// A cell's share of the liquid weight on a z-face, and the weight between
+// cells a (below) and b (src/mod_pressure_3d.f90:406-417).
+__device__ __forceinline__ double liq_share(const PPArgs& x, unsigned f, double al, double rho, double T) {
+    return ((f & ACT_L) ? 1.0 : 0.0) * al * rho * (1.0 - x.beta * (T - x.T_amb));
+}
+__device__ __forceinline__ double liq_weight(double share_a, double share_b) {
+    return 0.5 * GRAVITY * (share_a + share_b);
 }
 
 struct Pos {
@@ -168,6 +174,13 @@ __device__ __forceinline__ long at(const A& a, int i, int j, int k) {
     return (long)(i + 1) + a.sy * (j + 1) + a.sz * (k + 1);
 }
 
+__global__ __launch_bounds__(BLOCK) void k_pp_act(PPArgs a) {
+    const long o = cell_of_thread(a);
+    if (o >= a.n) return;
+    const CellAct c = cell_act(a, o);
+    a.act[o] = (unsigned char)((c.fluid ? ACT_FLUID : 0) | (c.l ? ACT_L : 0) | (c.g ? ACT_G : 0));
+}
+
 __global__ __launch_bounds__(BLOCK) void k_pp_grad(PPArgs a) {
     const long o = cell_of_thread(a);
     if (o >= a.n) return;
@@ -175,21 +188,22 @@ __global__ __launch_bounds__(BLOCK) void k_pp_grad(PPArgs a) {
     const int i = q.i, j = q.j, k = q.k;
     const bool interior = i >= 1 && i <= a.nr && j >= 1 && j <= a.nth && k >= 1 && k <= a.nz;
     double gr = 0.0, gth = 0.0, gz = 0.0, gzg = 0.0;
-    if (interior && a.ct[o] != 0) {
-        const long oW = at(a, i - 1, j, k), oE = at(a, i + 1, j, k);
-        const long oS = at(a, i, j - 1, k), oN = at(a, i, j + 1, k);
-        const long oB = at(a, i, j, k - 1), oT = at(a, i, j, k + 1);
-        const double* p = a.p;
+    if (interior && (a.act[o] & ACT_FLUID)) {
+        const long oW = o - 1, oE = o + 1, oS = o - a.sy, oN = o + a.sy, oB = o - a.sz, oT = o + a.sz;
+        const unsigned fo = a.act[o], fW = a.act[oW], fE = a.act[oE], fS = a.act[oS], fN = a.act[oN], fB = a.act[oB],
+                       fT = a.act[oT];
+        const double p0 = a.p[o], pW = a.p[oW], pE = a.p[oE], pS = a.p[oS], pN = a.p[oN], pB = a.p[oB], pT = a.p[oT];
+        const double so = liq_share(a, fo, a.al[o], a.rhol[o], a.Tl[o]);
+        const double sB = liq_share(a, fB, a.al[oB], a.rhol[oB], a.Tl[oB]);
+        const double sT = liq_share(a, fT, a.al[oT], a.rhol[oT], a.Tl[oT]);
         const double ri = a.r[i + 1];
-        const CellAct cW = cell_act(a, oW), cE = cell_act(a, oE), cS = cell_act(a, oS);
-        const CellAct cN = cell_act(a, oN), cB = cell_act(a, oB), cT = cell_act(a, oT);
-        gr = pgrad(p[oW], p[o], p[oE], a.r[i], a.r[i + 1], a.r[i + 2], i > 1 && pv_of(cW), i < a.nr && pv_of(cE));
-        gth = pgrad(p[oS], p[o], p[oN], ri * a.th[j], ri * a.th[j + 1], ri * a.th[j + 2], pv_of(cS), pv_of(cN));
-        const bool okm = k > 1 && pv_of(cB), okp = k < a.nz && pv_of(cT);
-        gz = pgrad(p[oB], p[o], p[oT], a.z[k], a.z[k + 1], a.z[k + 2], okm, okp);
+        gr = pgrad(pW, p0, pE, a.r[i], a.r[i + 1], a.r[i + 2], i > 1 && pv_of(fW), i < a.nr && pv_of(fE));
+        gth = pgrad(pS, p0, pN, ri * a.th[j], ri * a.th[j + 1], ri * a.th[j + 2], pv_of(fS), pv_of(fN));
+        const bool okm = k > 1 && pv_of(fB), okp = k < a.nz && pv_of(fT);
+        gz = pgrad(pB, p0, pT, a.z[k], a.z[k + 1], a.z[k + 2], okm, okp);
         double gb = 0.0, gt = 0.0;
-        if (okm) gb = (p[o] - p[oB]) / (a.z[k + 1] - a.z[k]) + liq_weight(a, oB, o);
-        if (okp) gt = (p[oT] - p[o]) / (a.z[k + 2] - a.z[k + 1]) + liq_weight(a, o, oT);
+        if (okm) gb = (p0 - pB) / (a.z[k + 1] - a.z[k]) + liq_weight(sB, so);
+        if (okp) gt = (pT - p0) / (a.z[k + 2] - a.z[k + 1]) + liq_weight(so, sT);
         gzg = okm && okp ? 0.5 * (gb + gt) : okp ? gt : okm ? gb : 0.0;
     }
     a.gr[o] = gr;
@@ -205,12 +219,15 @@ struct Phase {
     bool gas;
 };
 
-__device__ __forceinline__ bool face_open(const PPArgs& a, bool isg, double u_f, long neg, long pos) {
-    if (isg || !a.liq_room) return true;
-    if (u_f > 0.0 && a.liq_room[pos] <= ROOM_EPS) return false;
-    if (u_f < 0.0 && a.liq_room[neg] <= ROOM_EPS) return false;
-    return true;
-}
+// What both phases' face terms read of a cell and its neighbours, in the
+// order o, W, E, S, N, B, T.
+struct Around {
+    long at[7];
+    unsigned f[7];           // ACT_*
+    double vol[7], p[7], room[7];
+    double Ar_o, Ar_W, Ath, Az_o, Az_B;
+    double lw_B, lw_T;       // the liquid weight on the z-faces
+};
 
 struct Acc {
     double aW, aE, aS, aN, aB, aT, Su, flux;
@@ -218,107 +235,108 @@ struct Acc {
     int lk[3];
 };
 
+// Whether the liquid may pass the face from cell neg to cell pos (the room
+// on the side it flows to).
+__device__ __forceinline__ bool face_open(const PPArgs& a, bool isg, double u_f, double room_neg, double room_pos) {
+    if (isg || !a.liq_room) return true;
+    return !(u_f > 0.0 && room_pos <= ROOM_EPS) && !(u_f < 0.0 && room_neg <= ROOM_EPS);
+}
+
 // The six faces of cell o for one phase (src/mod_pressure_3d.f90:486-607).
-// nb: the activity of the neighbours W, E, S, N, B, T.
-__device__ void add_phase(const PPArgs& a, const Phase& ph, int i, int j, int k, long o, const CellAct* nb, Acc& c) {
+__device__ __forceinline__ void add_phase(const PPArgs& a, const Phase& ph, int i, int j, int k, const Around& n,
+                                          Acc& c) {
     const bool gas = ph.gas;
-    bool lk[6];
+    const unsigned mine = gas ? ACT_G : ACT_L;
+    enum { O, W, E, S, N, B, T };
+    const long o = n.at[O];
+    double al[7];
 #pragma unroll
-    for (int q = 0; q < 6; ++q) lk[q] = nb[q].fluid && (gas ? nb[q].g : nb[q].l);
-    const double* aef = ph.alpha;
-    const double* pf = a.p;
-    const long oW = at(a, i - 1, j, k), oE = at(a, i + 1, j, k);
-    const long oS = at(a, i, j - 1, k), oN = at(a, i, j + 1, k);
-    const long oB = at(a, i, j, k - 1), oT = at(a, i, j, k + 1);
+    for (int q = 0; q < 7; ++q) al[q] = ph.alpha[n.at[q]];
+    const double pr_o = ph.aPr[o], pr_W = ph.aPr[n.at[W]], pr_E = ph.aPr[n.at[E]];
+    const double pt_o = ph.aPth[o], pt_S = ph.aPth[n.at[S]], pt_N = ph.aPth[n.at[N]];
+    const double pz_o = ph.aPz[o], pz_B = ph.aPz[n.at[B]], pz_T = ph.aPz[n.at[T]];
+    const double ur_o = ph.ur[o], ur_W = ph.ur[n.at[W]], ur_E = ph.ur[n.at[E]];
+    const double ut_o = ph.uth[o], ut_S = ph.uth[n.at[S]], ut_N = ph.uth[n.at[N]];
+    const double uz_o = ph.uz[o], uz_B = ph.uz[n.at[B]], uz_T = ph.uz[n.at[T]];
+    const double gr_o = a.gr[o], gr_W = a.gr[n.at[W]], gr_E = a.gr[n.at[E]];
     // theta halos of the gradients: the periodic copies
-    const int js = j - 1 == 0 ? a.nth : j - 1, jn = j + 1 == a.nth + 1 ? 1 : j + 1;
-    const long gS = at(a, i, js, k), gN = at(a, i, jn, k);
-    const double* gr = a.gr;
-    const double* gth = a.gth;
-    const double* gz = ph.gz;
+    const long gS = j == 1 ? o + (long)(a.nth - 1) * a.sy : n.at[S], gN = j == a.nth ? o - (long)(a.nth - 1) * a.sy : n.at[N];
+    const double gt_o = a.gth[o], gt_S = a.gth[gS], gt_N = a.gth[gN];
+    const double gz_o = ph.gz[o], gz_B = ph.gz[n.at[B]], gz_T = ph.gz[n.at[T]];
+    // a cell's alpha vol / a_P^u in each direction
+    const double dr_o = al[O] * n.vol[O] / fmax(pr_o, SMALL), dt_o = al[O] * n.vol[O] / fmax(pt_o, SMALL),
+                 dz_o = al[O] * n.vol[O] / fmax(pz_o, SMALL);
     double d_f, af, u_f, delta;
-    if (lk[0]) {
-        d_f = 0.5 * (aef[o] * a.vol[o] / fmax(ph.aPr[o], SMALL) + aef[oW] * a.vol[oW] / fmax(ph.aPr[oW], SMALL));
-        af = 0.5 * (aef[o] + aef[oW]);
-        delta = a.r[i + 1] - a.r[i];
-        u_f = 0.5 * (ph.ur[oW] + ph.ur[o]) + d_f * (0.5 * (gr[oW] + gr[o]) - (pf[o] - pf[oW]) / delta);
-        if (face_open(a, gas, u_f, oW, o)) {
-            c.aW = c.aW + af * d_f * a.Ar[oW] / delta;
-            c.Su = c.Su + af * u_f * a.Ar[oW];
-            c.flux += fabs(af * u_f * a.Ar[oW]);
-        }
+    bool open;
+    d_f = 0.5 * (dr_o + al[W] * n.vol[W] / fmax(pr_W, SMALL));
+    af = 0.5 * (al[O] + al[W]);
+    delta = a.r[i + 1] - a.r[i];
+    u_f = 0.5 * (ur_W + ur_o) + d_f * (0.5 * (gr_W + gr_o) - (n.p[O] - n.p[W]) / delta);
+    open = (n.f[W] & ACT_FLUID) && (n.f[W] & mine) && face_open(a, gas, u_f, n.room[W], n.room[O]);
+    c.aW = open ? c.aW + af * d_f * n.Ar_W / delta : c.aW;
+    c.Su = open ? c.Su + af * u_f * n.Ar_W : c.Su;
+    c.flux = open ? c.flux + fabs(af * u_f * n.Ar_W) : c.flux;
+
+    d_f = 0.5 * (dr_o + al[E] * n.vol[E] / fmax(pr_E, SMALL));
+    af = 0.5 * (al[O] + al[E]);
+    delta = a.r[i + 2] - a.r[i + 1];
+    u_f = 0.5 * (ur_o + ur_E) + d_f * (0.5 * (gr_o + gr_E) - (n.p[E] - n.p[O]) / delta);
+    open = (n.f[E] & ACT_FLUID) && (n.f[E] & mine) && face_open(a, gas, u_f, n.room[O], n.room[E]);
+    c.aE = open ? c.aE + af * d_f * n.Ar_o / delta : c.aE;
+    c.Su = open ? c.Su - af * u_f * n.Ar_o : c.Su;
+    c.flux = open ? c.flux + fabs(af * u_f * n.Ar_o) : c.flux;
+    if (!gas) {
+        c.Fs[0] = open ? af * u_f * n.Ar_o : 0.0;
+        c.ac[0] = open ? af * d_f * n.Ar_o / delta : 0.0;
+        c.lk[0] = open ? 1 : 0;
     }
-    if (lk[1]) {
-        d_f = 0.5 * (aef[o] * a.vol[o] / fmax(ph.aPr[o], SMALL) + aef[oE] * a.vol[oE] / fmax(ph.aPr[oE], SMALL));
-        af = 0.5 * (aef[o] + aef[oE]);
-        delta = a.r[i + 2] - a.r[i + 1];
-        u_f = 0.5 * (ph.ur[o] + ph.ur[oE]) + d_f * (0.5 * (gr[o] + gr[oE]) - (pf[oE] - pf[o]) / delta);
-        if (face_open(a, gas, u_f, o, oE)) {
-            c.aE = c.aE + af * d_f * a.Ar[o] / delta;
-            c.Su = c.Su - af * u_f * a.Ar[o];
-            c.flux += fabs(af * u_f * a.Ar[o]);
-            if (!gas) {
-                c.Fs[0] = af * u_f * a.Ar[o];
-                c.ac[0] = af * d_f * a.Ar[o] / delta;
-                c.lk[0] = 1;
-            }
-        }
+
+    d_f = 0.5 * (dt_o + al[S] * n.vol[S] / fmax(pt_S, SMALL));
+    af = 0.5 * (al[O] + al[S]);
+    delta = a.r[i + 1] * (a.th[j + 1] - a.th[j]);
+    u_f = 0.5 * (ut_S + ut_o) + d_f * (0.5 * (gt_S + gt_o) - (n.p[O] - n.p[S]) / delta);
+    open = (n.f[S] & ACT_FLUID) && (n.f[S] & mine) && face_open(a, gas, u_f, n.room[S], n.room[O]);
+    c.aS = open ? c.aS + af * d_f * n.Ath / delta : c.aS;
+    c.Su = open ? c.Su + af * u_f * n.Ath : c.Su;
+    c.flux = open ? c.flux + fabs(af * u_f * n.Ath) : c.flux;
+
+    d_f = 0.5 * (dt_o + al[N] * n.vol[N] / fmax(pt_N, SMALL));
+    af = 0.5 * (al[O] + al[N]);
+    delta = a.r[i + 1] * (a.th[j + 2] - a.th[j + 1]);
+    u_f = 0.5 * (ut_o + ut_N) + d_f * (0.5 * (gt_o + gt_N) - (n.p[N] - n.p[O]) / delta);
+    open = (n.f[N] & ACT_FLUID) && (n.f[N] & mine) && face_open(a, gas, u_f, n.room[O], n.room[N]);
+    c.aN = open ? c.aN + af * d_f * n.Ath / delta : c.aN;
+    c.Su = open ? c.Su - af * u_f * n.Ath : c.Su;
+    c.flux = open ? c.flux + fabs(af * u_f * n.Ath) : c.flux;
+    if (!gas) {
+        c.Fs[1] = open ? af * u_f * n.Ath : 0.0;
+        c.ac[1] = open ? af * d_f * n.Ath / delta : 0.0;
+        c.lk[1] = open ? 1 : 0;
     }
-    if (lk[2]) {
-        d_f = 0.5 * (aef[o] * a.vol[o] / fmax(ph.aPth[o], SMALL) + aef[oS] * a.vol[oS] / fmax(ph.aPth[oS], SMALL));
-        af = 0.5 * (aef[o] + aef[oS]);
-        delta = a.r[i + 1] * (a.th[j + 1] - a.th[j]);
-        u_f = 0.5 * (ph.uth[oS] + ph.uth[o]) + d_f * (0.5 * (gth[gS] + gth[o]) - (pf[o] - pf[oS]) / delta);
-        if (face_open(a, gas, u_f, oS, o)) {
-            c.aS = c.aS + af * d_f * a.Ath[o] / delta;
-            c.Su = c.Su + af * u_f * a.Ath[o];
-            c.flux += fabs(af * u_f * a.Ath[o]);
-        }
-    }
-    if (lk[3]) {
-        d_f = 0.5 * (aef[o] * a.vol[o] / fmax(ph.aPth[o], SMALL) + aef[oN] * a.vol[oN] / fmax(ph.aPth[oN], SMALL));
-        af = 0.5 * (aef[o] + aef[oN]);
-        delta = a.r[i + 1] * (a.th[j + 2] - a.th[j + 1]);
-        u_f = 0.5 * (ph.uth[o] + ph.uth[oN]) + d_f * (0.5 * (gth[o] + gth[gN]) - (pf[oN] - pf[o]) / delta);
-        if (face_open(a, gas, u_f, o, oN)) {
-            c.aN = c.aN + af * d_f * a.Ath[o] / delta;
-            c.Su = c.Su - af * u_f * a.Ath[o];
-            c.flux += fabs(af * u_f * a.Ath[o]);
-            if (!gas) {
-                c.Fs[1] = af * u_f * a.Ath[o];
-                c.ac[1] = af * d_f * a.Ath[o] / delta;
-                c.lk[1] = 1;
-            }
-        }
-    }
-    if (lk[4]) {
-        d_f = 0.5 * (aef[o] * a.vol[o] / fmax(ph.aPz[o], SMALL) + aef[oB] * a.vol[oB] / fmax(ph.aPz[oB], SMALL));
-        af = 0.5 * (aef[o] + aef[oB]);
-        delta = a.z[k + 1] - a.z[k];
-        u_f = 0.5 * (ph.uz[oB] + ph.uz[o]) +
-              d_f * (0.5 * (gz[oB] + gz[o]) - (pf[o] - pf[oB]) / delta - (gas ? liq_weight(a, oB, o) : 0.0));
-        if (face_open(a, gas, u_f, oB, o)) {
-            c.aB = c.aB + af * d_f * a.Az[oB] / delta;
-            c.Su = c.Su + af * u_f * a.Az[oB];
-            c.flux += fabs(af * u_f * a.Az[oB]);
-        }
-    }
-    if (lk[5]) {
-        d_f = 0.5 * (aef[o] * a.vol[o] / fmax(ph.aPz[o], SMALL) + aef[oT] * a.vol[oT] / fmax(ph.aPz[oT], SMALL));
-        af = 0.5 * (aef[o] + aef[oT]);
-        delta = a.z[k + 2] - a.z[k + 1];
-        u_f = 0.5 * (ph.uz[o] + ph.uz[oT]) +
-              d_f * (0.5 * (gz[o] + gz[oT]) - (pf[oT] - pf[o]) / delta - (gas ? liq_weight(a, o, oT) : 0.0));
-        if (face_open(a, gas, u_f, o, oT)) {
-            c.aT = c.aT + af * d_f * a.Az[o] / delta;
-            c.Su = c.Su - af * u_f * a.Az[o];
-            c.flux += fabs(af * u_f * a.Az[o]);
-            if (!gas) {
-                c.Fs[2] = af * u_f * a.Az[o];
-                c.ac[2] = af * d_f * a.Az[o] / delta;
-                c.lk[2] = 1;
-            }
-        }
+
+    d_f = 0.5 * (dz_o + al[B] * n.vol[B] / fmax(pz_B, SMALL));
+    af = 0.5 * (al[O] + al[B]);
+    delta = a.z[k + 1] - a.z[k];
+    u_f = 0.5 * (uz_B + uz_o) +
+          d_f * (0.5 * (gz_B + gz_o) - (n.p[O] - n.p[B]) / delta - (gas ? n.lw_B : 0.0));
+    open = (n.f[B] & ACT_FLUID) && (n.f[B] & mine) && face_open(a, gas, u_f, n.room[B], n.room[O]);
+    c.aB = open ? c.aB + af * d_f * n.Az_B / delta : c.aB;
+    c.Su = open ? c.Su + af * u_f * n.Az_B : c.Su;
+    c.flux = open ? c.flux + fabs(af * u_f * n.Az_B) : c.flux;
+
+    d_f = 0.5 * (dz_o + al[T] * n.vol[T] / fmax(pz_T, SMALL));
+    af = 0.5 * (al[O] + al[T]);
+    delta = a.z[k + 2] - a.z[k + 1];
+    u_f = 0.5 * (uz_o + uz_T) +
+          d_f * (0.5 * (gz_o + gz_T) - (n.p[T] - n.p[O]) / delta - (gas ? n.lw_T : 0.0));
+    open = (n.f[T] & ACT_FLUID) && (n.f[T] & mine) && face_open(a, gas, u_f, n.room[O], n.room[T]);
+    c.aT = open ? c.aT + af * d_f * n.Az_o / delta : c.aT;
+    c.Su = open ? c.Su - af * u_f * n.Az_o : c.Su;
+    c.flux = open ? c.flux + fabs(af * u_f * n.Az_o) : c.flux;
+    if (!gas) {
+        c.Fs[2] = open ? af * u_f * n.Az_o : 0.0;
+        c.ac[2] = open ? af * d_f * n.Az_o / delta : 0.0;
+        c.lk[2] = open ? 1 : 0;
     }
 }
 
@@ -332,23 +350,41 @@ __global__ __launch_bounds__(BLOCK) void k_pp_assemble(PPArgs a) {
         const bool interior = i >= 1 && i <= a.nr && j >= 1 && j <= a.nth && k >= 1 && k <= a.nz;
         Acc c = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, {0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}, {0, 0, 0}};
         double aP = 0.0;
-        if (interior && a.ct[o] != 0) {
-            const bool al = act_l(a, o), ag = act_g(a, o);
-            const CellAct nb[6] = {cell_act(a, at(a, i - 1, j, k)), cell_act(a, at(a, i + 1, j, k)),
-                                   cell_act(a, at(a, i, j - 1, k)), cell_act(a, at(a, i, j + 1, k)),
-                                   cell_act(a, at(a, i, j, k - 1)), cell_act(a, at(a, i, j, k + 1))};
+        const unsigned fo = a.act[o];
+        if (interior && (fo & ACT_FLUID)) {
+            const bool al = fo & ACT_L, ag = fo & ACT_G;
+            Around n;
+            const long at7[7] = {o, o - 1, o + 1, o - a.sy, o + a.sy, o - a.sz, o + a.sz};
+#pragma unroll
+            for (int m = 0; m < 7; ++m) {
+                n.at[m] = at7[m];
+                n.f[m] = a.act[at7[m]];
+                n.vol[m] = a.vol[at7[m]];
+                n.p[m] = a.p[at7[m]];
+                n.room[m] = a.liq_room ? a.liq_room[at7[m]] : 1.0;
+            }
+            n.Ar_o = a.Ar[o];
+            n.Ar_W = a.Ar[o - 1];
+            n.Ath = a.Ath[o];
+            n.Az_o = a.Az[o];
+            n.Az_B = a.Az[o - a.sz];
+            n.lw_B = n.lw_T = 0.0;
+            const double al_o = a.al[o], rho_o = a.rhol[o];
             if (al) {
                 const Phase L = {a.al, a.url, a.uthl, a.uzl, a.aPrl, a.aPthl, a.aPzl, a.gz, false};
-                add_phase(a, L, i, j, k, o, nb, c);
+                add_phase(a, L, i, j, k, n, c);
             }
             if (a.two_phase && ag) {
+                const double so = liq_share(a, fo, al_o, rho_o, a.Tl[o]);
+                n.lw_B = liq_weight(liq_share(a, n.f[5], a.al[o - a.sz], a.rhol[o - a.sz], a.Tl[o - a.sz]), so);
+                n.lw_T = liq_weight(so, liq_share(a, n.f[6], a.al[o + a.sz], a.rhol[o + a.sz], a.Tl[o + a.sz]));
                 const Phase Gp = {a.ag, a.urg, a.uthg, a.uzg, a.aPrg, a.aPthg, a.aPzg, a.gzg, true};
-                add_phase(a, Gp, i, j, k, o, nb, c);
+                add_phase(a, Gp, i, j, k, n, c);
             }
             if (a.compress && ag) {
-                const double src = a.ag[o] * a.vol[o] / a.dt *
+                const double src = a.ag[o] * n.vol[0] / a.dt *
                                    (a.rhog[o] - a.rho_gas * a.T_amb / fmax(a.Toldg[o], T_MIN_GAS)) / fmax(a.rhog[o], SMALL);
-                const double cap = COMP_SRC_CAP * a.ag[o] * a.vol[o] / a.dt;
+                const double cap = COMP_SRC_CAP * a.ag[o] * n.vol[0] / a.dt;
                 c.Su = c.Su - fmax(-cap, fmin(cap, src));
             }
             if (!al && !ag) {
@@ -357,8 +393,8 @@ __global__ __launch_bounds__(BLOCK) void k_pp_assemble(PPArgs a) {
                 c.Su = 0.0;
             } else {
                 aP = (c.aW + c.aE + c.aS + c.aN + c.aB + c.aT) * (1.0 + PP_COMPLIANCE);
-                if (a.compress && ag) aP = aP + a.ag[o] / P0_THERMO * a.vol[o] / a.dt;
-                if (al) aP = aP + a.al[o] * a.vol[o] / (a.rhol[o] * (C_SOUND_LIQ * C_SOUND_LIQ) * a.dt);
+                if (a.compress && ag) aP = aP + a.ag[o] / P0_THERMO * n.vol[0] / a.dt;
+                if (al) aP = aP + al_o * n.vol[0] / (rho_o * (C_SOUND_LIQ * C_SOUND_LIQ) * a.dt);
             }
             // boundary rows (src/mod_boundary_3d.f90:218-275; serial: every boundary physical)
             const long sy2 = a.nr + 4;
@@ -376,10 +412,10 @@ __global__ __launch_bounds__(BLOCK) void k_pp_assemble(PPArgs a) {
                 aP = 1.0;
                 c.Su = 0.0;
             } else {
-                if (i > 1 && a.ct[at(a, i - 1, j, k)] == 0) c.aW = 0.0;
-                if (i < a.nr && a.ct[at(a, i + 1, j, k)] == 0) c.aE = 0.0;
-                if (k > 1 && a.ct[at(a, i, j, k - 1)] == 0) c.aB = 0.0;
-                if (k < a.nz && a.ct[at(a, i, j, k + 1)] == 0) c.aT = 0.0;
+                if (i > 1 && !(n.f[1] & ACT_FLUID)) c.aW = 0.0;
+                if (i < a.nr && !(n.f[2] & ACT_FLUID)) c.aE = 0.0;
+                if (k > 1 && !(n.f[5] & ACT_FLUID)) c.aB = 0.0;
+                if (k < a.nz && !(n.f[6] & ACT_FLUID)) c.aT = 0.0;
                 if (k == a.nz) {
                     if (outlet(i - 1, j)) c.aW = 0.0;
                     if (outlet(i + 1, j)) c.aE = 0.0;
@@ -556,7 +592,11 @@ struct PPWork {
     hipStream_t stream = nullptr;
     DevBuf<double> coord, f3, grads, outs, part, room, exd;
     DevBuf<int> ct, outlet, masks, lki;
-    std::vector<double> part_h;
+    DevBuf<unsigned char> act;       // k_pp_act's bytes
+    double* part_h = nullptr;        // pinned: the blocks' sums
+    ~PPWork() {
+        if (part_h) (void)hipHostFree(part_h);
+    }
 };
 
 std::mutex g_pp_mutex;
@@ -573,6 +613,7 @@ int ensure_pp(const eafp_desc* d) {
     EAFP_TRY_RC(w.coord.alloc((size_t)(d->nr + d->ntheta + d->nz + 12)));
     EAFP_TRY_RC(w.f3.alloc((size_t)n * NF3));
     EAFP_TRY_RC(w.grads.alloc((size_t)n * 4));
+    EAFP_TRY_RC(w.act.alloc((size_t)n));
     EAFP_TRY_RC(w.outs.alloc((size_t)n * 8));
     EAFP_TRY_RC(w.room.alloc((size_t)n));
     EAFP_TRY_RC(w.ct.alloc((size_t)n));
@@ -582,7 +623,9 @@ int ensure_pp(const eafp_desc* d) {
     EAFP_TRY_RC(w.lki.alloc((size_t)n * 6));
     const long blocks = pp_blocks(n, (long)(d->nr + 4) * (d->ntheta + 4));
     EAFP_TRY_RC(w.part.alloc((size_t)blocks * 2));
-    w.part_h.assign((size_t)blocks * 2, 0.0);
+    if (w.part_h) (void)hipHostFree(w.part_h);
+    w.part_h = nullptr;
+    EAFP_TRY(hipHostMalloc((void**)&w.part_h, sizeof(double) * 2 * blocks, hipHostMallocDefault));
     w.nr = d->nr;
     w.nth = d->ntheta;
     w.nz = d->nz;
@@ -741,8 +784,10 @@ int pp_assemble(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_confi
     a.gth = w.grads.p + n;
     a.gz = w.grads.p + 2 * n;
     a.gzg = w.grads.p + 3 * n;
+    a.act = w.act.p;
     a.part = w.part.p;
     const int blocks = pp_blocks(n, a.sz);
+    k_pp_act<<<blocks, BLOCK, 0, w.stream>>>(a);
     k_pp_grad<<<blocks, BLOCK, 0, w.stream>>>(a);
     k_pp_assemble<<<blocks, BLOCK, 0, w.stream>>>(a);
     EAFP_TRY(hipGetLastError());
@@ -757,7 +802,7 @@ int pp_assemble(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_confi
                 EAFP_TRY(hipMemcpyAsync(ex_i[q], w.lki.p + (long)q * n, sizeof(int) * n, D2H, w.stream));
         }
     }
-    EAFP_TRY(hipMemcpyAsync(w.part_h.data(), w.part.p, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost, w.stream));
+    EAFP_TRY(hipMemcpyAsync(w.part_h, w.part.p, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost, w.stream));
     EAFP_TRY(hipStreamSynchronize(w.stream));
     double fl = 0.0, su = 0.0;
     for (int b = 0; b < blocks; ++b) {
@@ -898,19 +943,20 @@ int pp_correct(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_config
 // Allocation-free assembly (eafp_pp_assemble_noalloc).  The kernels' scratch
 // -- the four gradient arrays and the continuity residual's block partials
 // and sums -- lives in `scratch`, a static device array of the library sized
-// for EAFP_NOALLOC_MAX_CELLS padded cells (32.5 MiB; each GPU the library
+// for EAFP_NOALLOC_MAX_CELLS padded cells (33.5 MiB; each GPU the library
 // runs on holds one until the process ends).  Host code never names the
 // array itself, only its device address from hipGetSymbolAddress, taken
 // once per device with that device current.  Every call on a GPU shares its
 // array, which keeps the last call's contents: the kernels write every
-// value they later read (every padded cell's gradients, every block's
-// partials), so nothing needs clearing; calls that overlap on one GPU race.
+// value they later read (every padded cell's gradients and activity byte,
+// every block's partials), so nothing needs clearing; calls that overlap on one GPU race.
 // ---------------------------------------------------------------------------
 namespace {
 
 constexpr long NA_CELLS = EAFP_NOALLOC_MAX_CELLS;
 constexpr long NA_BLOCKS = 32768;                        // block partial pairs
-constexpr long NA_DOUBLES = 4 * NA_CELLS + 2 * NA_BLOCKS + 32;   // gradients, partials, the two sums (padded)
+constexpr long NA_DOUBLES = 4 * NA_CELLS + 2 * NA_BLOCKS + 32 + NA_CELLS / 8;   // gradients, partials, the two sums
+                                                                               // (padded), activity bytes
 static_assert(NA_DOUBLES % 32 == 0, "256-byte multiple");
 
 static __device__ __align__(256) double scratch[NA_DOUBLES];
@@ -985,6 +1031,8 @@ int pp_assemble_noalloc(const eafp_desc* d, const eafp_pp_fields* f, const eafp_
     a.gzg = sc + 3 * n;
     a.part = sc + 4 * NA_CELLS;
     double* sums = a.part + 2 * NA_BLOCKS;
+    a.act = reinterpret_cast<unsigned char*>(sums + 32);
+    k_pp_act<<<(int)blocks, BLOCK, 0, stream>>>(a);
     k_pp_grad<<<(int)blocks, BLOCK, 0, stream>>>(a);
     k_pp_assemble<<<(int)blocks, BLOCK, 0, stream>>>(a);
     k_pp_partsum<<<1, BLOCK, 0, stream>>>(a.part, (int)blocks, sums);

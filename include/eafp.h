@@ -189,7 +189,7 @@ int eafp_pp_assemble(const eafp_desc* desc, const eafp_pp_fields* fields, const 
  * block sums are reduced on the device in the same order), but no
  * hipMalloc, hipFree or other allocating call: the kernels' scratch (the
  * cell gradients, the residual's block sums) is a static device array of
- * the library, 32.5 MiB held by each GPU the library runs on until the
+ * the library, 33.5 MiB held by each GPU the library runs on until the
  * process ends.  Meshes beyond EAFP_NOALLOC_MAX_CELLS padded cells:
  * EAFP_ERR_SIZE.  Runs on `stream` (a hipStream_t; NULL: the default
  * stream) and returns synchronised; residual and flux_ref are host
