@@ -28,11 +28,11 @@
 //                  pivots m(e) and c'(e) of the forward elimination (they
 //                  depend on the coefficients only), the chain kernel's
 //                  records, the end terms and the wall halo lines
-//   k_tdma_prep<P> and k_tdma_chain<P>: the pass on one work-group per system,
-//                  the lines of a diagonal on the lanes of the chain waves
-//                  (the schedule is described in tdma_line.hpp); it runs a
-//                  pass wherever chain_plan admits it and the pass's pivots
-//                  are in its division's band
+//   k_tdma_prep<P> and k_tdma_chain: a pass, or a part of one, on one
+//                  work-group per system, the lines of a diagonal on the
+//                  lanes of the chain waves (the schedule is described in
+//                  tdma_line.hpp); it runs a pass wherever chain_plan admits
+//                  it and the pass's pivots are in its division's band
 //   k_tdma_pass<P> the other passes: one 1024-thread work-group per system: per
 //                  diagonal, all threads stage d(e) (the right-hand side from
 //                  the neighbour lines, whose indices follow from the
@@ -51,7 +51,13 @@
 // A single system is latency-bound by design: one CU walks the
 // (nth+nz-1) + (nr+nz-1) + (nr+nth-1) diagonals of a sweep, each a chain of
 // dependent FP64 steps; independent systems (the equations of one time
-// step) run on other CUs side by side.
+// step) run on other CUs side by side.  What bounds a diagonal is the LDS that
+// feeds the chain: an element takes about 80 cycles of it forward and 26 back
+// (a wave's access of 16 bytes a lane 4 cycles read and 13 written, of 8 bytes
+// 8 and 8), against 35 and 17 of the recurrences alone.  So the passes of a
+// sweep overlap where one can start before the other ends (chain_part),
+// side by side in one launch: two sweeps of 60x120x84 with the packing and the
+// setup take 8.31 ms instead of 9.87.
 //
 // Built without floating-point contraction, with the reference's operand
 // order, so every value of phi is the double the sequential loops compute.
@@ -147,12 +153,15 @@ __global__ __launch_bounds__(TD_PASS_BLOCK) void k_tdma_pass(const TdSys* __rest
 }
 
 // The per-pass products of the chain kernel's records (prep_elem), one
-// thread per element of every line.
+// thread per element of every line of the part (prep_part).
 template <int P>
-__global__ __launch_bounds__(TD_BLOCK) void k_tdma_prep(const TdSys* __restrict__ sys) {
-    const TdPass& p = sys[blockIdx.y].ps[P];
+__global__ __launch_bounds__(TD_BLOCK) void k_tdma_prep(const TdSys* __restrict__ sys, int part, int parts) {
+    const TdSys& s = sys[blockIdx.y];
+    const TdPass& p = s.ps[P];
     const long t = (long)blockIdx.x * TD_BLOCK + threadIdx.x;
-    if (t < (long)p.n * p.NL) prep_elem<P>(p, (int)(t % p.NL), (int)(t / p.NL));
+    if (t >= (long)p.n * p.NL) return;
+    const int l = (int)(t % p.NL);
+    if (parts == 1 || in_prep_part(s, P, p.uv[l], part, parts)) prep_elem<P>(p, l, (int)(t / p.NL));
 }
 
 // One forward chunk f for a helper lane: issue the loads of chunk f+2 into
@@ -160,17 +169,17 @@ __global__ __launch_bounds__(TD_BLOCK) void k_tdma_prep(const TdSys* __restrict_
 // barriers of the phases up to the one before f's, read the same chunk of
 // the diagonal before from the x slots (the chain overwrites it next), fill
 // f's ring slot from `use` (loaded two chunks ago), store the copy to phi,
-// and close the phase.  Past the pass's last chunk
-// (`live` false, the same for every lane) and on the first diagonal the
+// and close the phase (phases count from the part's first, ph0).  Past the
+// part's last chunk (`live` false, the same for every lane) and on the first diagonal the
 // copies go to the sink, and past the last chunk nothing is filled and no
 // barrier passed.  Every call issues the same stores and loads, so the
 // compiler's waits for `use` count exactly the accesses issued after it; a
 // wave whose entries all lie past the chunk (h0, its first lane's h, is
 // uniform) skips the fill and the copy's LDS read.
 template <int P, int IPL>
-__device__ __forceinline__ void helper_chunk(const TdPass& p, const TdLds& L, long& X, TdTask& f, TdTask& fl, int h,
+__device__ __forceinline__ void helper_chunk(const TdPass& p, const TdLds& L, long& X, long ph0, TdTask& f, TdTask& fl, int h,
                                              int h0, int HL, bool live, const TdPre (&use)[IPL], TdPre (&next)[IPL]) {
-    const long ph = chain_prep_phase(p, f);
+    const long ph = chain_prep_phase(p, f) - ph0;
     // chunk fl's loads first: they depend on nothing this phase does, and
     // they drain through the memory pipeline while the fill and the copy run
     // (with three entries per lane the registers do not allow it)
@@ -212,27 +221,30 @@ __device__ __forceinline__ void helper_chunk(const TdPass& p, const TdLds& L, lo
     chain_advance_fwd(p, fl);
 }
 
-// One pass of one system per work-group (the schedule is described in
-// tdma_line.hpp): the first NW waves run the recurrences at raised wave
-// priority, the other waves feed them, IPL ring entries per helper lane and
-// chunk (at least the pass's p.IPL).  Every wave passes the same number of
-// barriers, one per phase and one after the x slots' initial ones; the
-// branch between the two roles is uniform per wave.
+// A part of one pass of one system (the schedule is described in
+// tdma_line.hpp, the parts at chain_part): the first NW waves run the
+// recurrences at raised wave priority, the other waves feed them, IPL ring
+// entries per helper lane and chunk (the pass's p.IPL).  Every wave passes
+// the same number of barriers, one per phase and those after the x slots'
+// initial values; the branch between the two roles is uniform per wave.
 template <int P, int IPL>
-__global__ __launch_bounds__(TDC_BLOCK) void k_tdma_chain(const TdSys* __restrict__ sys) {
-    __shared__ __align__(16) double lds[TDC_LDS];
-    if (sys[blockIdx.x].off_band[P]) return;    // a pivot outside the band: k_tdma_pass runs this pass
-    const TdPass p = sys[blockIdx.x].ps[P];     // by value: its fields stay in scalar registers
+__device__ __forceinline__ void chain_run(const TdSys& s, const TdSpan& span, double* lds) {
+    const TdPass p = s.ps[P];     // by value: its fields stay in scalar registers
     const TdLds L = chain_lds(p, lds);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const long nph = chain_phases(p);
+    const long nph = (long)(span.hi - span.lo) * (p.K + 2), ph0 = (long)span.lo * (p.K + 2);
     chain_init_slots(p, L, (int)threadIdx.x, TDC_BLOCK);
     __syncthreads();
+    const TdTask begin = chain_at(p, span.lo);
+    if (span.lo > 0) {      // the part before left the x of its last diagonal in phi
+        for (int it = (int)threadIdx.x; it < p.n * begin.pm; it += TDC_BLOCK) chain_take_up(p, L, begin, it);
+        __syncthreads();
+    }
     if (wave < p.NW) {
         __builtin_amdgcn_s_setprio(3);
         const int j = (int)threadIdx.x;
         double dp = 0.0;
-        TdTask t = chain_first(p);
+        TdTask t = begin;
         for (long X = 0; X < nph; ++X) {
             if (t.kind == 1) chain_forward(p, L, t, (int)(X & 1), j, dp);
             else if (t.kind == 2) chain_backward(p, L, t, j);
@@ -242,9 +254,12 @@ __global__ __launch_bounds__(TDC_BLOCK) void k_tdma_chain(const TdSys* __restric
         __builtin_amdgcn_s_setprio(0);
     } else {
         const int HL = TDC_BLOCK - 64 * p.NW, h = (int)threadIdx.x - 64 * p.NW, h0 = 64 * (wave - p.NW);
-        const long nf = (long)(p.nu + p.nv - 1) * p.K;     // forward chunks of the pass
+        const long nf = (long)(span.hi - span.lo) * p.K;   // forward chunks of the part
         TdPre r0[IPL], r1[IPL], r2[IPL];
-        TdTask f = chain_first_fwd(p), fl = f;
+        TdTask f = begin;
+        f.idx = 1;
+        chain_set_kind(p, f);
+        TdTask fl = f;
 #pragma unroll
         for (int i = 0; i < IPL; ++i) chain_load<P>(p, fl, h + i * HL, r0[i]);
         chain_advance_fwd(p, fl);
@@ -253,35 +268,60 @@ __global__ __launch_bounds__(TDC_BLOCK) void k_tdma_chain(const TdSys* __restric
         chain_advance_fwd(p, fl);
         long X = 0;
         for (long q = 0; q < nf; q += 3) {
-            helper_chunk<P, IPL>(p, L, X, f, fl, h, h0, HL, true, r0, r2);
-            helper_chunk<P, IPL>(p, L, X, f, fl, h, h0, HL, q + 1 < nf, r1, r0);
-            helper_chunk<P, IPL>(p, L, X, f, fl, h, h0, HL, q + 2 < nf, r2, r1);
+            helper_chunk<P, IPL>(p, L, X, ph0, f, fl, h, h0, HL, true, r0, r2);
+            helper_chunk<P, IPL>(p, L, X, ph0, f, fl, h, h0, HL, q + 1 < nf, r1, r0);
+            helper_chunk<P, IPL>(p, L, X, ph0, f, fl, h, h0, HL, q + 2 < nf, r2, r1);
         }
         for (; X < nph; ++X) __syncthreads();
     }
     // the last diagonal's x, after the last barrier
-    TdTask t = chain_first(p);
-    for (int w = 0; w < p.nu + p.nv - 2; ++w) chain_next_diagonal(p, t);
+    const TdTask t = chain_at(p, span.hi - 1);
     const int cnt = p.n * t.m;
     for (int it = (int)threadIdx.x; it < cnt; it += TDC_BLOCK)
         chain_copy_out(p, L, true, t.w, t.v_lo, t.m, t.mM, t.l0, 0, p.n, it);
 }
 
-template <int P>
-void launch_chain(int ipl, int nsys, hipStream_t st, const TdSys* tp) {
-    if (ipl <= 1) k_tdma_chain<P, 1><<<nsys, TDC_BLOCK, 0, st>>>(tp);
-    else if (ipl == 2) k_tdma_chain<P, 2><<<nsys, TDC_BLOCK, 0, st>>>(tp);
-    else k_tdma_chain<P, 3><<<nsys, TDC_BLOCK, 0, st>>>(tp);
+// A launch's passes, first .. first + gridDim.y - 1, and the part of each.
+struct TdStage {
+    int first, part[3], parts;
+};
+
+// One part per work-group, gridDim.y passes of every system side by side.
+__global__ __launch_bounds__(TDC_BLOCK) void k_tdma_chain(const TdSys* __restrict__ sys, TdStage g) {
+    __shared__ __align__(16) double lds[TDC_LDS];
+    const TdSys& s = sys[blockIdx.x];
+    const int P = g.first + (int)blockIdx.y;
+    if (s.off_band[P]) return;    // a pivot outside the band: k_tdma_pass runs this pass
+    const TdSpan span = chain_part(s, P, g.part[P], g.parts);
+    if (span.lo >= span.hi) return;
+    switch (P * TDC_IPL + s.ps[P].IPL) {
+    case 1: chain_run<0, 1>(s, span, lds); return;
+    case 2: chain_run<0, 2>(s, span, lds); return;
+    case 3: chain_run<0, 3>(s, span, lds); return;
+    case 4: chain_run<1, 1>(s, span, lds); return;
+    case 5: chain_run<1, 2>(s, span, lds); return;
+    case 6: chain_run<1, 3>(s, span, lds); return;
+    case 7: chain_run<2, 1>(s, span, lds); return;
+    case 8: chain_run<2, 2>(s, span, lds); return;
+    case 9: chain_run<2, 3>(s, span, lds); return;
+    }
+}
+static_assert(TDC_IPL == 3, "k_tdma_chain dispatches 1 to 3 entries per lane");
+
+// Pass P alone, whole.
+void launch_chain(int P, int nsys, hipStream_t st, const TdSys* tp) {
+    k_tdma_chain<<<nsys, TDC_BLOCK, 0, st>>>(tp, TdStage{P, {0, 0, 0}, 1});
 }
 
-// One tile of one system per work-group (move_tile_*).
+// One tile of one system per work-group (move_tile_*), those of the part.
 template <int P, int Q>
-__global__ __launch_bounds__(TD_PACK_BLOCK) void k_tdma_move(const TdSys* __restrict__ sys) {
+__global__ __launch_bounds__(TD_PACK_BLOCK) void k_tdma_move(const TdSys* __restrict__ sys, int part, int parts) {
     __shared__ double buf[TD_PT3];
     __shared__ int order[2][TD_PT * TD_PT], lidx[2][TD_PT * TD_PT];
     const TdSys& s = sys[blockIdx.y];
     PackTile t;
     if (!pack_tile_of(s, blockIdx.x, t)) return;     // the whole work-group
+    if (parts > 1 && !in_move_part(s, P, t, part, parts)) return;
     const int tid = (int)threadIdx.x;
     pack_tile_order(s, P, t, order[0], lidx[0], tid, TD_PACK_BLOCK);
     if (Q < 3) pack_tile_order(s, Q, t, order[1], lidx[1], tid, TD_PACK_BLOCK);
@@ -297,8 +337,16 @@ __global__ __launch_bounds__(TD_BLOCK) void k_tdma_wall_halo(const TdSys* __rest
     if (t < (long)(s.nr + 4) * (s.nz + 4)) wall_halo_column(s, t);
 }
 
+// Of a call whose passes overlap: parts per pass, the largest number of
+// systems, and the fewest steps that have to be hidden (overlap_pays).
+constexpr int TD_PARTS = 4;
+constexpr int TD_OVERLAP_SYS = 16;
+constexpr long TD_OVERLAP_STEPS = 3200;
+
 struct TdWork {
     hipStream_t stream = nullptr;
+    int* off_h = nullptr;      // pinned: off_band of every system
+    size_t off_n = 0;
     DevBuf<double> work;       // packed arrays and pass copies of phi of every system
     DevBuf<int> iwork;         // diagonal starts
     DevBuf<double> stage;      // host arrays: 9 padded arrays per system
@@ -315,6 +363,34 @@ void pass_shape(const eafp_desc& d, int P, int& nu, int& nv, int& n) {
     else { nu = d.nr; nv = d.ntheta; n = d.nz; }
 }
 
+// Whether overlapped sweeps pay.  What they can hide is the last nz - 1
+// diagonals of the r pass and the last nr - 1 of the theta pass, so many
+// elements in a row; what they cost is eighteen more launches and the parts'
+// starts.  Three sweeps of one system, overlapped against in turn: with 1184
+// steps to hide (17x40x33) 1.90 ms against 1.77, with 3065 (35x50x40) 3.17
+// against 3.18, with 3924 (35x66x49) 4.10 against 4.37 and with 12060
+// (60x120x84) 12.3 against 14.7.  A batch gains less, as the moves and the
+// products of its parts take longer than their launches: 16 systems of
+// 35x66x49 5.17 against 5.17 and of 60x120x84 19.1 against 20.0, 32 of them
+// 6.19 against 5.92 and 25.3 against 24.7.
+bool overlap_pays(int nsys, const eafp_desc* d) {
+    long steps = 0;
+    for (int q = 0; q < nsys; ++q)
+        steps = std::max(steps, (long)(d[q].nz - 1) * d[q].nr + (long)(d[q].nr - 1) * d[q].ntheta);
+    return nsys <= TD_OVERLAP_SYS && steps >= TD_OVERLAP_STEPS;
+}
+
+// off_h for n flags.
+int ensure_flags(TdWork& w, size_t n) {
+    if (w.off_n >= n) return EAFP_OK;
+    if (w.off_h) (void)hipHostFree(w.off_h);
+    w.off_h = nullptr;
+    w.off_n = 0;
+    EAFP_TRY(hipHostMalloc((void**)&w.off_h, sizeof(int) * n, hipHostMallocDefault));
+    w.off_n = n;
+    return EAFP_OK;
+}
+
 int halo_lines(int P, int nu, int nv) { return P == 0 ? 2 * nu + nv : P == 1 ? 2 * nv + 2 * nu : 2 * nv + nu; }
 
 }  // namespace
@@ -326,7 +402,6 @@ int tdma_solve_batch(int nsys, const eafp_desc* descs, const eafp_tdma_system* s
     // EAFP_TDMA_KERNEL=pass keeps k_tdma_pass for every pass.
     const char* force = std::getenv("EAFP_TDMA_KERNEL");
     bool chain[3] = {true, true, true};
-    int ipl[3] = {1, 1, 1};     // the chain kernel's ring entries per helper lane: the most any system needs
     if (force && std::strcmp(force, "pass") == 0) chain[0] = chain[1] = chain[2] = false;
     for (int q = 0; q < nsys; ++q)
         for (int P = 0; P < 3; ++P) {
@@ -336,7 +411,6 @@ int tdma_solve_batch(int nsys, const eafp_desc* descs, const eafp_tdma_system* s
             t.NH = halo_lines(P, t.nu, t.nv);
             t.NLX = t.NL + t.NH;
             if (!chain_plan(t, 1 << 20)) chain[P] = false;
-            else ipl[P] = std::max(ipl[P], t.IPL);
         }
     for (int q = 0; q < nsys; ++q) {
         EAFP_TRY_RC(validate_desc(&descs[q]));
@@ -356,7 +430,7 @@ int tdma_solve_batch(int nsys, const eafp_desc* descs, const eafp_tdma_system* s
             iwork += nu + nv - 1 + (chain[P] ? NL : 0);
             lines += NL;
         }
-        iwork += 3;     // off_band flags
+        iwork += 3;     // off_band flags, every system's first
         stage += 9 * (long)(d.nr + 4) * (d.ntheta + 4) * (d.nz + 4);
         max_lines = std::max(max_lines, lines);
         max_cells = std::max(max_cells, ncells);
@@ -377,7 +451,7 @@ int tdma_solve_batch(int nsys, const eafp_desc* descs, const eafp_tdma_system* s
     std::vector<int> ihost((size_t)iwork);
     double* dcur = w.work.p;
     int* icur = w.iwork.p;
-    long ioff = 0, soff = 0;
+    long ioff = 3L * nsys, soff = 0;
     for (int q = 0; q < nsys; ++q) {
         const eafp_desc& d = descs[q];
         const eafp_tdma_system& y = sys[q];
@@ -405,8 +479,7 @@ int tdma_solve_batch(int nsys, const eafp_desc* descs, const eafp_tdma_system* s
             EAFP_TRY(hipMemcpyAsync((void*)t.home, y.phi, sizeof(double) * t.n, hipMemcpyHostToDevice, w.stream));
             soff += 9 * t.n;
         }
-        t.off_band = (decltype(t.off_band))(icur + ioff);   // three zeros of ihost: cleared by the upload below
-        ioff += 3;
+        t.off_band = (decltype(t.off_band))(icur + 3L * q);   // three zeros of ihost: cleared by the upload below
         for (int P = 0; P < 3; ++P) {
             TdPass& p = t.ps[P];
             pass_shape(d, P, p.nu, p.nv, p.n);
@@ -455,28 +528,57 @@ int tdma_solve_batch(int nsys, const eafp_desc* descs, const eafp_tdma_system* s
     const dim3 g_tiles((unsigned)max_tiles, ny);
     k_tdma_pack<<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp);
     k_tdma_setup<<<g_lines, TD_BLOCK, 0, w.stream>>>(tp);
-    for (int sweep = 0; sweep < n_sweep; ++sweep) {
+    // Overlapped sweeps, where every pass of every system runs the chain kernel,
+    // which the setup decides last
+    bool overlap = chain[0] && chain[1] && chain[2] && overlap_pays(nsys, descs);
+    if (overlap) {
+        EAFP_TRY_RC(ensure_flags(w, 3 * (size_t)nsys));
+        EAFP_TRY(hipMemcpyAsync(w.off_h, icur, sizeof(int) * 3 * nsys, hipMemcpyDeviceToHost, w.stream));
+        EAFP_TRY(hipStreamSynchronize(w.stream));
+        for (int q = 0; q < 3 * nsys; ++q) overlap = overlap && !w.off_h[q];
+    }
+    for (int sweep = 0; sweep < n_sweep && overlap; ++sweep) {
+        // r part a beside theta part a - 1, theta part C + c beside z part c;
+        // between the launches a portion of planes or columns is handed on
+        const int C = TD_PARTS;
+        k_tdma_prep<0><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp, 0, 1);
+        for (int a = 0; a <= 2 * C; ++a) {
+            const int first = a < C ? 0 : a < 2 * C ? 1 : 2, last = a == 0 ? 0 : a <= C ? 1 : 2;
+            k_tdma_chain<<<dim3((unsigned)nsys, (unsigned)(last - first + 1)), TDC_BLOCK, 0, w.stream>>>(
+                tp, TdStage{first, {a, a - 1, a - C - 1}, C});
+            if (a < C) {
+                k_tdma_move<0, 1><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, a, C);
+                k_tdma_prep<1><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp, a, C);
+            } else if (a < 2 * C) {
+                k_tdma_move<1, 2><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, a - C, C);
+                k_tdma_prep<2><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp, a - C, C);
+            }
+        }
+        if (sweep + 1 < n_sweep) k_tdma_move<2, 0><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, 0, 1);
+        else k_tdma_move<2, 3><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, 0, 1);
+    }
+    for (int sweep = 0; sweep < n_sweep && !overlap; ++sweep) {
         // with the chain kernel planned, k_tdma_pass still runs the systems whose
         // pivots leave its band (each kernel returns at once for the others)
         if (chain[0]) {
-            k_tdma_prep<0><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp);
-            launch_chain<0>(ipl[0], nsys, w.stream, tp);
+            k_tdma_prep<0><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp, 0, 1);
+            launch_chain(0, nsys, w.stream, tp);
         }
         k_tdma_pass<0><<<nsys, TD_PASS_BLOCK, 0, w.stream>>>(tp);
-        k_tdma_move<0, 1><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp);
+        k_tdma_move<0, 1><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, 0, 1);
         if (chain[1]) {
-            k_tdma_prep<1><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp);
-            launch_chain<1>(ipl[1], nsys, w.stream, tp);
+            k_tdma_prep<1><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp, 0, 1);
+            launch_chain(1, nsys, w.stream, tp);
         }
         k_tdma_pass<1><<<nsys, TD_PASS_BLOCK, 0, w.stream>>>(tp);
-        k_tdma_move<1, 2><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp);
+        k_tdma_move<1, 2><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, 0, 1);
         if (chain[2]) {
-            k_tdma_prep<2><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp);
-            launch_chain<2>(ipl[2], nsys, w.stream, tp);
+            k_tdma_prep<2><<<g_cells, TD_BLOCK, 0, w.stream>>>(tp, 0, 1);
+            launch_chain(2, nsys, w.stream, tp);
         }
         k_tdma_pass<2><<<nsys, TD_PASS_BLOCK, 0, w.stream>>>(tp);
-        if (sweep + 1 < n_sweep) k_tdma_move<2, 0><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp);
-        else k_tdma_move<2, 3><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp);
+        if (sweep + 1 < n_sweep) k_tdma_move<2, 0><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, 0, 1);
+        else k_tdma_move<2, 3><<<g_tiles, TD_PACK_BLOCK, 0, w.stream>>>(tp, 0, 1);
     }
     k_tdma_wall_halo<<<g_cols, TD_BLOCK, 0, w.stream>>>(tp);
     EAFP_TRY(hipGetLastError());
@@ -493,6 +595,7 @@ void tdma_release() {
     if (g_td) {
         if (g_td->stream) (void)hipStreamSynchronize(g_td->stream);
         if (g_td->stream) (void)hipStreamDestroy(g_td->stream);
+        if (g_td->off_h) (void)hipHostFree(g_td->off_h);
         delete g_td;
         g_td = nullptr;
     }

@@ -977,6 +977,89 @@ __host__ __device__ inline long chain_phases(const TdPass& p) { return (long)(p.
 
 __host__ __device__ inline int chain_slot(const TdPass& p, int u, int v) { return p.by_u ? u - 1 : v - 1; }
 
+// The parts of a sweep whose passes overlap.  The r pass (k outer) is done
+// with plane k when its diagonal nth + k - 2 is, and theta line (i,k) reads
+// planes k and k+1 only; the theta pass is done with column i when its
+// diagonal nz + i - 2 is, and z line (i,j) reads columns i and i+1 only.  So
+// planes, then columns, are handed on in `parts` portions of whole tiles,
+// portion c the planes (columns) td_bound(c) + 1 .. td_bound(c+1):
+//   r pass, part c          up to the diagonal that completes portion c
+//   k_tdma_move, k_tdma_prep  portion c of the planes, and the lines that
+//                           need nothing beyond them
+//   theta pass, part c      the diagonals of prepared lines; from the last
+//                           portion on (part parts-1) cut where portions of
+//                           the columns are complete: 2 parts - 1 parts
+//   z pass, part c          as the theta pass on portion c of the columns
+// A diagonal's lines need nothing of their own pass but the diagonal before,
+// so a part starts from the x that the part before has left in phi.
+struct TdSpan {
+    int lo, hi;          // diagonals lo .. hi-1
+};
+
+__host__ __device__ inline int td_bound(int n, int c, int parts) {
+    const int tiles = (n + TD_PT - 1) / TD_PT, whole = parts * (parts + 1);
+    const int b = (tiles * c * (c + 1) + whole - 1) / whole * TD_PT;
+    return b < n ? b : n;
+}
+
+// Lines with the handed-on coordinate up to this are prepared once portions
+// 0 .. c-1 have been handed on.
+__host__ __device__ inline int td_prepared(int n, int c, int parts) {
+    const int b = td_bound(n, c, parts);
+    return b == n ? n : b > 0 ? b - 1 : 0;
+}
+
+// The end of part c-1, and so the start of part c, of pass P.
+__host__ __device__ inline int chain_part_end(const TdSys& s, int P, int c, int parts) {
+    if (c == 0) return 0;
+    if (P == 0) {
+        const int b = td_bound(s.nz, c, parts);
+        return b > 0 ? s.nth + b - 1 : 0;
+    }
+    if (P == 1) return c < parts ? td_prepared(s.nz, c, parts) : s.nz + td_bound(s.nr, c - parts + 1, parts) - 1;
+    return c < parts ? td_prepared(s.nr, c, parts) : s.nr + s.nth - 1;
+}
+
+__host__ __device__ inline TdSpan chain_part(const TdSys& s, int P, int c, int parts) {
+    return TdSpan{chain_part_end(s, P, c, parts), chain_part_end(s, P, c + 1, parts)};
+}
+
+// Whether the line with uv = u | v << 16 of pass 1 or 2 is prepared in part c,
+// and whether a tile's cells are moved out of pass 0 or 1 in part c.
+__host__ __device__ inline bool in_prep_part(const TdSys& s, int P, int uv, int c, int parts) {
+    const int n = P == 1 ? s.nz : s.nr, x = P == 1 ? uv >> 16 : uv & 0xffff;
+    return x > td_prepared(n, c, parts) && x <= td_prepared(n, c + 1, parts);
+}
+__host__ __device__ inline bool in_move_part(const TdSys& s, int P, const PackTile& t, int c, int parts) {
+    const int n = P == 0 ? s.nz : s.nr, x = P == 0 ? t.k0 : t.i0;
+    return x >= td_bound(n, c, parts) && x < td_bound(n, c + 1, parts);
+}
+
+// Phase G of diagonal w.
+__host__ __device__ inline TdTask chain_at(const TdPass& p, int w) {
+    TdTask t = chain_first(p);
+    if (w > 0) {
+        t.w = w - 1;
+        int hi;
+        diagonal_range(w - 1, p.nu, p.nv, t.v_lo, hi);
+        t.m = hi - t.v_lo + 1;
+        t.mM = td_magic((unsigned)t.m);
+        t.l0 = p.dstart[w - 1];
+        chain_next_diagonal(p, t);
+        chain_set_kind(p, t);
+    }
+    return t;
+}
+
+// Entry `it` of the x of the diagonal before t's, from the pass's phi into
+// its x slot.
+__host__ __device__ inline void chain_take_up(const TdPass& p, const TdLds& L, const TdTask& t, int it) {
+    int e, j;
+    td_divmod(it, t.pm, t.pmM, e, j);
+    const int v = t.pv_lo + j, u = t.w + 1 - v;
+    L.xb[td_mul24(chain_slot(p, u, v), L.LS) + e] = p.phi[(unsigned)(td_mul24(e, p.NLX) + t.pl0 + j)];
+}
+
 // What a helper lane loads for one ring entry: the record.
 struct TdPre {
     double r[RC_N];
