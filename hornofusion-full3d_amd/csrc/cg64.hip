@@ -507,7 +507,7 @@ static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* s
     *done = 0;
     EAFP_TRY(hipEventRecord(w->t0, B.stream));
     EAFP_TRY_RC(start_resident64(B, w->slot1.p, w->cst.p, tol, max_iter));
-    const ResidentGate held(D.plan.T > 1 ? D.plan.nteam * D.plan.T : 0);
+    const ResidentGate held(D.plan.members);
     for (;;) {
         EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, RES_ITERS));
         EAFP_TRY_RC(download_all(B, w->x.p));
@@ -596,7 +596,7 @@ int time_resident64(Batch& B, int iters, float* ms) {
     Cg64Work* w = B.cg64;
     if (!w->res || w->res->given_up) return EAFP_OK;
     ResDevice& D = *w->res;
-    const ResidentGate held(D.plan.T > 1 ? D.plan.nteam * D.plan.T : 0);
+    const ResidentGate held(D.plan.members);
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
         EAFP_TRY_RC(start_resident64(B, w->slot1.p, w->cst.p, 0.0, 1 << 30));
         EAFP_TRY(hipEventRecord(w->t0, B.stream));

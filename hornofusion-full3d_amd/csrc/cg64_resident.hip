@@ -68,11 +68,8 @@ __global__ __launch_bounds__(RB, 2) void k64_resident(R64Args g) {
     const int tid = threadIdx.x;
     Team t;
     int team;
-    res_member((int)blockIdx.x, g.L.nteam, g.L.T, team, t.m);
-    if (team >= g.L.nteam) return;
+    if (!res_place(g.L, team, t.m, t.T, t.slots)) return;
     if (!res_gate(g.L, S)) return;
-    t.T = g.L.T;
-    t.slots = g.L.slots + (size_t)team * 2 * t.T * SLOT_WORDS;
     t.gate = g.L.gate;
     t.tag = uniform(g.L.gate[1]);
     const Cg64Args& a = g.a;
@@ -381,7 +378,7 @@ int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int
     g.L = D.launch();
     g.zx = zx;
     g.iters = iters;
-    const size_t lds = std::max(p.lds, p.T > 1 ? (size_t)RES_LDS_ALONE : (size_t)0);
+    const size_t lds = std::max(p.lds, p.members > 0 ? (size_t)RES_LDS_ALONE : (size_t)0);
     switch (p.slots) {
         case 1: return launch_u<1>(g, p.blocks, lds, B.stream);
         case 2: return launch_u<2>(g, p.blocks, lds, B.stream);

@@ -1957,7 +1957,7 @@ static int launch_resident_mixed(Batch& B, int fmt, int interval) {
     g.L = w->res->launch();
     g.xz = w->xz.p;
     g.interval = interval;
-    const size_t lds = std::max(p.lds, p.T > 1 ? (size_t)RES_LDS_ALONE : (size_t)0);
+    const size_t lds = std::max(p.lds, p.members > 0 ? (size_t)RES_LDS_ALONE : (size_t)0);
     const bool line = w->args.line != 0;
     if (fmt == EAFP_COEF_BF16) return rmx_launch_bf16(line, w->res_cq, p.slots, g, p.blocks, lds, B.stream);
     if (fmt == EAFP_COEF_FP16) return rmx_launch_fp16(line, w->res_cq, p.slots, g, p.blocks, lds, B.stream);
@@ -2117,7 +2117,7 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
     int given_up = 0;
     if (B.resident_mixed && w->res && !w->res->given_up) {
         const ResPlan& p = w->res->plan;
-        const ResidentGate held(p.T > 1 ? p.nteam * p.T : 0);
+        const ResidentGate held(p.members);
         EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, true, &given_up));
         w->res->given_up = given_up != 0;
     } else {
@@ -2168,7 +2168,7 @@ int time_resident_mixed(Batch& B, int fmt, int precond, int iters, float* ms) {
     w->args.line = precond == EAFP_PRECOND_ZLINE ? 1 : 0;
     ResDevice& D = *w->res;
     EAFP_TRY_RC(rmx_prepare(fmt, w->args.line != 0, w->res_cq, D.plan.slots));
-    const ResidentGate held(D.plan.T > 1 ? D.plan.nteam * D.plan.T : 0);
+    const ResidentGate held(D.plan.members);
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
         EAFP_TRY_RC(mixed_start(B, o, fmt));
         EAFP_TRY_RC(D.arm(resident_tags(D, iters), B.stream));

@@ -207,11 +207,8 @@ __global__ __launch_bounds__(RB, 2) void k_mresident(RMxArgs g) {
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
     Team t;
     int team;
-    res_member((int)blockIdx.x, g.L.nteam, g.L.T, team, t.m);
-    if (team >= g.L.nteam) return;
+    if (!res_place(g.L, team, t.m, t.T, t.slots)) return;
     if (!res_gate(g.L, S)) return;
-    t.T = g.L.T;
-    t.slots = g.L.slots + (size_t)team * 2 * t.T * SLOT_WORDS;
     t.gate = g.L.gate;
     t.tag = uniform(g.L.gate[1]);
     const MxArgs& a = g.a;

@@ -62,13 +62,22 @@ struct ResItem {
     long xoff;          // first element of the system in the exchange buffer
 };
 
-// A launch: teams of T work-groups; team t takes the items
+// A team of a launch whose teams differ in size: its work-groups and the
+// first slot of its own.
+struct ResTeam {
+    int T, slot0;
+};
+
+// A launch: teams of T work-groups, or (T = 0) of the sizes of `teams`, with
+// the team and member of each work-group in `member`; team t takes the items
 // [team_begin[t], team_begin[t+1]) one after another.
 struct ResLaunch {
     const ResItem* items;
     const int* team_begin;
+    const ResTeam* teams;
+    const int2* member;
     int nteam, T;
-    u64* slots;         // nteam * 2 * T * SLOT_WORDS
+    u64* slots;         // 2 * T * SLOT_WORDS of every team
     unsigned* gate;     // [0] arrivals and the give-up mark, [1] the next launch's first tag
     int expected;       // work-groups that pass the gate
     int pad_;
@@ -181,6 +190,26 @@ __host__ __device__ __forceinline__ void res_member(int b, int nteam, int T, int
 // ---------------------------------------------------------------------------
 // Device side
 // ---------------------------------------------------------------------------
+// The team and member of this work-group; false when it has none.
+__device__ __forceinline__ bool res_place(const ResLaunch& L, int& team, int& m, int& T, u64*& slots) {
+    int slot0;
+    if (L.T) {
+        res_member((int)blockIdx.x, L.nteam, L.T, team, m);
+        if (team >= L.nteam) return false;
+        T = L.T;
+        slot0 = team * 2 * T;
+    } else {
+        const int2 b = L.member[blockIdx.x];
+        team = __builtin_amdgcn_readfirstlane(b.x);
+        m = __builtin_amdgcn_readfirstlane(b.y);
+        if (team < 0) return false;
+        T = __builtin_amdgcn_readfirstlane(L.teams[team].T);
+        slot0 = __builtin_amdgcn_readfirstlane(L.teams[team].slot0);
+    }
+    slots = L.slots + (size_t)slot0 * SLOT_WORDS;
+    return true;
+}
+
 __device__ __forceinline__ u64 ld_agent(const u64* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }

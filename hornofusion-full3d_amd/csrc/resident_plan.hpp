@@ -21,13 +21,17 @@ struct ResLimits {
 struct ResPlan {
     bool ok = false;
     int nsys = 0;
-    int T = 0, nteam = 0, blocks = 0;
+    int T = 0, nteam = 0, blocks = 0;         // T = 0: teams of different sizes
+    int members = 0;                          // work-groups that wait for each other (0: teams of one)
     int slots = 0;                            // largest over the items
     size_t lds = 0;
     int max_items = 0;                        // longest team list
     float est_us = 0.f;                       // model: one iteration of every system
     std::vector<ResItem> items;               // team by team
     std::vector<int> team_begin;
+    std::vector<ResTeam> teams;               // with T = 0
+    std::vector<int2> member;
+    int nslot = 0;                            // slots of all teams
     long xlen = 0;                            // elements of the exchange buffer
 };
 
@@ -55,6 +59,8 @@ struct ResDevice {
     ResPlan plan;
     DevBuf<ResItem> items;
     DevBuf<int> team_begin;
+    DevBuf<ResTeam> teams;
+    DevBuf<int2> member;
     DevBuf<u64> slots;
     DevBuf<unsigned> gate;
     unsigned tag = 1;             // first tag of the next launch
