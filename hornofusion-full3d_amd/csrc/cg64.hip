@@ -371,13 +371,10 @@ static int init_cg64(Batch& B, Cg64Work* w) {
         EAFP_TRY(hipMemset(w->p0.p, 0, n * sizeof(double)));
         EAFP_TRY(hipMemset(w->p1.p, 0, n * sizeof(double)));
         ResPlan plan = plan_resident64(B);
-        if (plan.ok) {
-            auto d = std::make_unique<ResDevice>();
-            EAFP_TRY_RC(w->zx.alloc(plan.xlen));
+        EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, w->zx, B.stream));
+        if (w->res) {
             EAFP_TRY(hipHostMalloc((void**)&w->slots_host, sizeof(CgSlot) * B.nsys, hipHostMallocDefault));
             EAFP_TRY(hipHostMalloc((void**)&w->gate_host, sizeof(unsigned), hipHostMallocDefault));
-            EAFP_TRY_RC(d->init(std::move(plan), B.stream));
-            w->res = std::move(d);
         }
     }
     return EAFP_OK;
@@ -600,7 +597,7 @@ int time_resident64(Batch& B, int iters, float* ms) {
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
         EAFP_TRY_RC(start_resident64(B, w->slot1.p, w->cst.p, 0.0, 1 << 30));
         EAFP_TRY(hipEventRecord(w->t0, B.stream));
-        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, iters));
+        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, std::min(iters, RES_ITERS)));
         EAFP_TRY(hipEventRecord(w->t1, B.stream));
         EAFP_TRY(hipMemcpyAsync(w->slots_host, w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));
         EAFP_TRY(hipMemcpyAsync(w->gate_host, D.gate.p, sizeof(unsigned), hipMemcpyDeviceToHost, B.stream));

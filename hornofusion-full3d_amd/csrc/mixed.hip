@@ -1781,12 +1781,7 @@ static int init_mixed(Batch& B, MixedWork* w) {
         EAFP_TRY(hipEventCreate(&w->t0));
         EAFP_TRY(hipEventCreate(&w->t1));
         ResPlan plan = plan_resident_mixed(B, &w->res_cq);
-        if (plan.ok) {
-            auto d = std::make_unique<ResDevice>();
-            EAFP_TRY_RC(w->xz.alloc(plan.xlen));
-            EAFP_TRY_RC(d->init(std::move(plan), B.stream));
-            w->res = std::move(d);
-        }
+        EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, w->xz, B.stream));
     }
     return EAFP_OK;
 }
@@ -1946,6 +1941,7 @@ static int rmx_prepare(int fmt, bool line, int cq, int slots) {
 }
 
 // Tags that one resident launch of `interval` inner iterations uses at most.
+constexpr long RES_STEP_TAGS = 1L << 28;
 static long resident_tags(const ResDevice& D, int interval) { return D.plan.max_items * (2L * interval + 2); }
 
 // The inner iterations of one refinement step, on chip.
@@ -2115,7 +2111,9 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
     interval = (interval + 1) & ~1;    // even: the p buffer parity restarts every step
     EAFP_TRY(hipEventRecord(w->t0, B.stream));
     int given_up = 0;
-    if (B.resident_mixed && w->res && !w->res->given_up) {
+    // a step's tags have to fit the 32 bits several times over (resident.hpp);
+    // longer steps, of millions of iterations, stream
+    if (B.resident_mixed && w->res && !w->res->given_up && resident_tags(*w->res, interval) < RES_STEP_TAGS) {
         const ResPlan& p = w->res->plan;
         const ResidentGate held(p.members);
         EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, true, &given_up));

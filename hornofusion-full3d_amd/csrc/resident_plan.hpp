@@ -1,6 +1,7 @@
 // resident_plan.hpp -- host side of the resident solvers: which batches
 // they take, the teams, and the launch's device tables.
 #pragma once
+#include <memory>
 #include <vector>
 
 #include "batch.hpp"
@@ -67,6 +68,23 @@ struct ResDevice {
     bool given_up = false;        // a launch did not get its CUs: stream from now on
     int init(ResPlan&& p, hipStream_t stream);
     ResLaunch launch() const;
+    // `out` and its exchange buffer; both stay empty, and the batch streams,
+    // where the plan is not ok or the device's memory does not hold them
+    template <typename X>
+    static int create(ResPlan&& p, std::unique_ptr<ResDevice>& out, DevBuf<X>& exchange, hipStream_t stream) {
+        if (!p.ok) return EAFP_OK;
+        auto d = std::make_unique<ResDevice>();
+        int rc = exchange.alloc(p.xlen);
+        if (rc == EAFP_OK) rc = d->init(std::move(p), stream);
+        if (rc == EAFP_OK) {
+            out = std::move(d);
+            return EAFP_OK;
+        }
+        exchange.release();
+        if (rc != (int)hipErrorOutOfMemory) return rc;
+        (void)hipGetLastError();
+        return EAFP_OK;
+    }
     // gate open and `tag` set for the next launch, which uses at most `tags` of them
     int arm(long tags, hipStream_t stream);
 };
