@@ -590,10 +590,10 @@ __global__ __launch_bounds__(BLOCK) void k_pp_seal(PCArgs a) {
 struct PPWork {
     int nr = -1, nth = -1, nz = -1;
     hipStream_t stream = nullptr;
-    DevBuf<double> coord, f3, grads, outs, part, room, exd;
+    DevBuf<double> coord, f3, grads, outs, room, exd;
     DevBuf<int> ct, outlet, masks, lki;
     DevBuf<unsigned char> act;       // k_pp_act's bytes
-    double* part_h = nullptr;        // pinned: the blocks' sums
+    double* part_h = nullptr;        // pinned: the blocks' sums, which the kernel stores there itself
     ~PPWork() {
         if (part_h) (void)hipHostFree(part_h);
     }
@@ -622,7 +622,6 @@ int ensure_pp(const eafp_desc* d) {
     EAFP_TRY_RC(w.exd.alloc((size_t)n * 6));
     EAFP_TRY_RC(w.lki.alloc((size_t)n * 6));
     const long blocks = pp_blocks(n, (long)(d->nr + 4) * (d->ntheta + 4));
-    EAFP_TRY_RC(w.part.alloc((size_t)blocks * 2));
     if (w.part_h) (void)hipHostFree(w.part_h);
     w.part_h = nullptr;
     EAFP_TRY(hipHostMalloc((void**)&w.part_h, sizeof(double) * 2 * blocks, hipHostMallocDefault));
@@ -785,7 +784,7 @@ int pp_assemble(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_confi
     a.gz = w.grads.p + 2 * n;
     a.gzg = w.grads.p + 3 * n;
     a.act = w.act.p;
-    a.part = w.part.p;
+    EAFP_TRY(hipHostGetDevicePointer((void**)&a.part, w.part_h, 0));
     const int blocks = pp_blocks(n, a.sz);
     k_pp_act<<<blocks, BLOCK, 0, w.stream>>>(a);
     k_pp_grad<<<blocks, BLOCK, 0, w.stream>>>(a);
@@ -802,7 +801,6 @@ int pp_assemble(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_confi
                 EAFP_TRY(hipMemcpyAsync(ex_i[q], w.lki.p + (long)q * n, sizeof(int) * n, D2H, w.stream));
         }
     }
-    EAFP_TRY(hipMemcpyAsync(w.part_h, w.part.p, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost, w.stream));
     EAFP_TRY(hipStreamSynchronize(w.stream));
     double fl = 0.0, su = 0.0;
     for (int b = 0; b < blocks; ++b) {

@@ -127,6 +127,22 @@ struct CompInfo {
 enum { CTR_UPLOADS = 0, CTR_LABELLED, CTR_CAPTURES, CTR_LAUNCHES, CTR_COUNT };
 void counter_add(int which, long long v);
 
+// Pinned memory that the caller's host arrays cross through in pieces, so that
+// one piece is on the link while the next is copied (batch.hip).
+struct HostRing {
+    static constexpr int SLOTS = 3;
+    static constexpr long SLOT_LEN = 1L << 18;       // doubles of a slot at most: 2 MiB
+    double* mem = nullptr;
+    long len = 0;                                    // doubles of a slot
+    hipEvent_t ev[SLOTS] = {};                       // behind the last copy from or to the slot
+    int next = 0;
+    bool none = false;                               // there is no pinned memory: the arrays go as they are
+    ~HostRing();
+    bool open(long want);                            // slots of `want` doubles, at most SLOT_LEN
+    int send(double* dst, const double* const* src, int nsrc, long n, hipStream_t st);
+    int receive(double* dst, const double* src, long n, hipStream_t st);
+};
+
 // One system of the download launch (batch.hip, k_phi_out).
 struct PhiOut {
     int nr, nth, nz;
@@ -171,6 +187,7 @@ struct Batch {
     long phi_blocks = 0;
     std::vector<char> uploaded;          // 0: no; 1: yes; 2: yes, singular components labelled
     DevBuf<double> staging;              // padded staging for uploads
+    HostRing ring;                       // host arrays cross through it
     DevBuf<int> lab;                     // component labelling: a cell index per cell
     DevBuf<unsigned char> lab_bits;      // link, anchor and root bits per cell
     DevBuf<int> lab_small;               // per-system flags, root lists and counts
@@ -187,11 +204,18 @@ struct Batch {
     int set_tiling(int cells_per_thread, int blocks);
     int set_columns(int r_splits);
     int upload_tables();
-    int upload(int s, const double* const host[8], const double* phi0, int arrays_on_device);
-    int download(int s, double* phi_host, int to_device);
+    // `wait` false: returns with the copies and the pack under way on `stream`;
+    // the caller's arrays stay as they are until the stream has been waited for
+    int upload(int s, const double* const host[8], const double* phi0, int arrays_on_device, bool wait = true);
+    int download(int s, double* phi_host, int to_device, bool wait = true);
     // labels the singular components of the systems uploaded since their
     // last labelling (only the mixed solver needs them)
     int label_components();
+    long longest_pad() const {
+        long n = 0;
+        for (int s = 0; s < nsys; ++s) n = std::max(n, padded_len(s));
+        return n;
+    }
     long padded_len(int s) const {
         const SysGeom& g = geom[s];
         return (long)(g.nr + 4) * (g.nth + 4) * (g.nz + 4);

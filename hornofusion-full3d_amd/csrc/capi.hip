@@ -68,9 +68,14 @@ int eafp_cg_solve(const eafp_desc* desc, const double* aW, const double* aE, con
     }
     eafp::Batch& B = g_cache->B;
     const double* arr[8] = {aW, aE, aS, aN, aB, aT, aP, Su};
-    if ((rc = B.upload(0, arr, phi, 0)) != EAFP_OK) return rc;
+    // one wait, behind the solve; whatever fails, nothing reads the caller's
+    // arrays after the return
     eafp_stats st{};
-    if ((rc = eafp::solve_fp64(B, max_iter, tol, &st, 0)) != EAFP_OK) return rc;
+    if ((rc = B.upload(0, arr, phi, 0, false)) == EAFP_OK) rc = eafp::solve_fp64(B, max_iter, tol, &st, 0);
+    if (rc != EAFP_OK) {
+        (void)hipStreamSynchronize(B.stream);
+        return rc;
+    }
     if ((rc = B.download(0, phi, 0)) != EAFP_OK) return rc;
     *residual = st.residual;
     *n_iter = st.n_iter;

@@ -52,8 +52,9 @@ struct Cg64Work {
 };
 
 ResPlan plan_resident64(const Batch& B);
-int start_resident64(Batch& B, CgSlot* slot, CgConst* cst, double tol, int max_iter);
-int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int iters);
+int start_resident64(Batch& B, ResDevice& D, CgSlot* slot, CgConst* cst, double tol, int max_iter, int iters);
+int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int iters, bool first);
+int report_resident64(Batch& B, ResDevice& D, const CgSlot* slot, CgSlot* slots_host, unsigned* gate_host);
 
 void free_cg64(Cg64Work* w) {
     if (!w) return;
@@ -503,14 +504,13 @@ static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* s
     ResDevice& D = *w->res;
     *done = 0;
     EAFP_TRY(hipEventRecord(w->t0, B.stream));
-    EAFP_TRY_RC(start_resident64(B, w->slot1.p, w->cst.p, tol, max_iter));
+    EAFP_TRY_RC(start_resident64(B, D, w->slot1.p, w->cst.p, tol, max_iter, RES_ITERS));
     const ResidentGate held(D.plan.members);
-    for (;;) {
-        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, RES_ITERS));
+    for (bool first = true;; first = false) {
+        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, RES_ITERS, first));
         EAFP_TRY_RC(download_all(B, w->x.p));
         EAFP_TRY(hipEventRecord(w->t1, B.stream));
-        EAFP_TRY(hipMemcpyAsync(w->slots_host, w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));
-        EAFP_TRY(hipMemcpyAsync(w->gate_host, D.gate.p, sizeof(unsigned), hipMemcpyDeviceToHost, B.stream));
+        EAFP_TRY_RC(report_resident64(B, D, w->slot1.p, w->slots_host, w->gate_host));
         EAFP_TRY(hipStreamSynchronize(B.stream));
         if (*w->gate_host & GATE_GIVEN_UP) {
             D.given_up = true;
@@ -594,13 +594,13 @@ int time_resident64(Batch& B, int iters, float* ms) {
     if (!w->res || w->res->given_up) return EAFP_OK;
     ResDevice& D = *w->res;
     const ResidentGate held(D.plan.members);
+    iters = std::min(iters, RES_ITERS);
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
-        EAFP_TRY_RC(start_resident64(B, w->slot1.p, w->cst.p, 0.0, 1 << 30));
+        EAFP_TRY_RC(start_resident64(B, D, w->slot1.p, w->cst.p, 0.0, 1 << 30, iters));
         EAFP_TRY(hipEventRecord(w->t0, B.stream));
-        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, std::min(iters, RES_ITERS)));
+        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, iters, true));
         EAFP_TRY(hipEventRecord(w->t1, B.stream));
-        EAFP_TRY(hipMemcpyAsync(w->slots_host, w->slot1.p, sizeof(CgSlot) * B.nsys, hipMemcpyDeviceToHost, B.stream));
-        EAFP_TRY(hipMemcpyAsync(w->gate_host, D.gate.p, sizeof(unsigned), hipMemcpyDeviceToHost, B.stream));
+        EAFP_TRY_RC(report_resident64(B, D, w->slot1.p, w->slots_host, w->gate_host));
         EAFP_TRY(hipStreamSynchronize(B.stream));
     }
     if (*w->gate_host & GATE_GIVEN_UP) {

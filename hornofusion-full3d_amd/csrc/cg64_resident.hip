@@ -352,9 +352,15 @@ static int launch_u(const R64Args& g, int blocks, size_t lds, hipStream_t st) {
     return EAFP_OK;
 }
 
-// Fresh slots and the solve's constants for every system.
-__global__ void k64_res_start(CgSlot* slot, CgConst* cst, int nsys, double tol, int max_iter) {
+// Fresh slots and the solve's constants for every system; opens the first
+// launch's gate.
+__global__ void k64_res_start(CgSlot* slot, CgConst* cst, int nsys, double tol, int max_iter, unsigned* gate,
+                              unsigned tag) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) {
+        gate[0] = 0;
+        gate[1] = tag;
+    }
     if (s >= nsys) return;
     CgSlot n{};
     n.bnorm = -1.0;
@@ -362,17 +368,40 @@ __global__ void k64_res_start(CgSlot* slot, CgConst* cst, int nsys, double tol, 
     cst[s] = CgConst{tol, max_iter, 0};
 }
 
-int start_resident64(Batch& B, CgSlot* slot, CgConst* cst, double tol, int max_iter) {
-    k64_res_start<<<(B.nsys + 255) / 256, 256, 0, B.stream>>>(slot, cst, B.nsys, tol, max_iter);
+static long launch_tags(const ResDevice& D, int iters) { return (long)D.plan.max_items * (2L * iters + 2); }
+
+int start_resident64(Batch& B, ResDevice& D, CgSlot* slot, CgConst* cst, double tol, int max_iter, int iters) {
+    unsigned tag = 0;
+    EAFP_TRY_RC(D.take_tags(launch_tags(D, iters), B.stream, &tag));
+    k64_res_start<<<(B.nsys + 255) / 256, 256, 0, B.stream>>>(slot, cst, B.nsys, tol, max_iter, D.gate.p, tag);
+    EAFP_TRY(hipGetLastError());
+    return EAFP_OK;
+}
+
+// The slots and the gate word, straight into the host's memory: one launch
+// instead of two copies.
+__global__ void k64_res_report(const CgSlot* slot, const unsigned* gate, int nsys, CgSlot* out, unsigned* gate_out) {
+    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+    if (s == 0) *gate_out = gate[0];
+    if (s < nsys) out[s] = slot[s];
+}
+
+int report_resident64(Batch& B, ResDevice& D, const CgSlot* slot, CgSlot* slots_host, unsigned* gate_host) {
+    CgSlot* out = nullptr;
+    unsigned* gate_out = nullptr;
+    EAFP_TRY(hipHostGetDevicePointer((void**)&out, slots_host, 0));
+    EAFP_TRY(hipHostGetDevicePointer((void**)&gate_out, gate_host, 0));
+    k64_res_report<<<(B.nsys + 255) / 256, 256, 0, B.stream>>>(slot, D.gate.p, B.nsys, out, gate_out);
     EAFP_TRY(hipGetLastError());
     return EAFP_OK;
 }
 
 // One launch: at most `iters` iterations of every unfinished system.  The
 // slots, x0, b, fold and the coefficients are the streaming kernels' own.
-int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int iters) {
+// `first`: start_resident64 has opened the gate.
+int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int iters, bool first) {
     const ResPlan& p = D.plan;
-    EAFP_TRY_RC(D.arm((long)p.max_items * (2L * iters + 2), B.stream));
+    if (!first) EAFP_TRY_RC(D.arm(launch_tags(D, iters), B.stream));
     R64Args g{};
     g.a = a;
     g.L = D.launch();

@@ -267,14 +267,21 @@ __global__ void k_res_arm(unsigned* gate, unsigned tag) {
     gate[1] = tag;
 }
 
-int ResDevice::arm(long tags, hipStream_t stream) {
+int ResDevice::take_tags(long tags, hipStream_t stream, unsigned* first) {
     if ((unsigned long)tag + (unsigned long)tags > 0xF0000000ul) {   // before the tags wrap, forget the old ones
         EAFP_TRY(hipMemsetAsync(slots.p, 0, sizeof(u64) * slots.n, stream));
         tag = 1;
     }
-    k_res_arm<<<1, 1, 0, stream>>>(gate.p, tag);
-    EAFP_TRY(hipGetLastError());
+    *first = tag;
     tag += (unsigned)tags;
+    return EAFP_OK;
+}
+
+int ResDevice::arm(long tags, hipStream_t stream) {
+    unsigned first = 0;
+    EAFP_TRY_RC(take_tags(tags, stream, &first));
+    k_res_arm<<<1, 1, 0, stream>>>(gate.p, first);
+    EAFP_TRY(hipGetLastError());
     return EAFP_OK;
 }
 

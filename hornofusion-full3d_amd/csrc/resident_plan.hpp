@@ -87,6 +87,8 @@ struct ResDevice {
     }
     // gate open and `tag` set for the next launch, which uses at most `tags` of them
     int arm(long tags, hipStream_t stream);
+    // the first of `tags` tags, for a kernel that opens the gate itself
+    int take_tags(long tags, hipStream_t stream, unsigned* first);
 };
 
 __global__ void k_res_arm(unsigned* gate, unsigned tag);

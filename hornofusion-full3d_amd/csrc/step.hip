@@ -185,26 +185,30 @@ int pp_step(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_config* c
     const double* csys[8];
     for (int q = 0; q < 8; ++q) csys[q] = sys[q];
     const bool mixed = o->solver == EAFP_STEP_MIXED;
-    EAFP_TRY_RC(B.upload(0, csys, nullptr, 1));
+    eafp_stats st{};
+    int rc = B.upload(0, csys, nullptr, 1, false);
     // launch shape by solver, as tuned on the 60x120x84 production mesh: the
     // FP64 CG at one cell per thread, the mixed solver at two; four blocks
     // per CU, at most one per tile
     const int cpt = mixed ? 2 : 1;
-    if (B.cpt != cpt) {
+    if (rc == EAFP_OK && B.cpt != cpt) {
         const int tiles = (int)((n_interior(d) + (long)BLOCK * cpt - 1) / ((long)BLOCK * cpt));
-        EAFP_TRY_RC(B.set_tiling(cpt, std::min(4 * device_cus(), tiles)));
+        rc = B.set_tiling(cpt, std::min(4 * device_cus(), tiles));
     }
-    eafp_stats st{};
-    if (mixed)
-        EAFP_TRY_RC(solve_mixed(B, o->mixed, &st));
-    else
-        EAFP_TRY_RC(solve_fp64(B, o->max_iter, o->tol, &st, 0));
+    if (rc == EAFP_OK) rc = mixed ? solve_mixed(B, o->mixed, &st) : solve_fp64(B, o->max_iter, o->tol, &st, 0);
+    if (rc != EAFP_OK) {
+        (void)hipStreamSynchronize(B.stream);   // the pack may still read the system
+        return rc;
+    }
     if (st.residual != st.residual) res = st.residual;   // :322
 
-    // the post-solve steps (:324-397), p' read from the solver's iterate
+    // the post-solve steps (:324-397) read p' from the solver's iterate; its copy
+    // to the caller runs beside them
     const double* ppd = B.phi_pad[0]->p;
-    EAFP_TRY_RC(pp_correct(d, &fdev, cfg, o->alpha_p, ppd, &ex, &iodev, 1));
-    EAFP_TRY_RC(B.download(0, pp, on_device));
+    EAFP_TRY_RC(B.download(0, pp, on_device, false));
+    rc = pp_correct(d, &fdev, cfg, o->alpha_p, ppd, &ex, &iodev, 1);
+    EAFP_TRY(hipStreamSynchronize(B.stream));
+    EAFP_TRY_RC(rc);
 
     if (!on_device) {
         const hipMemcpyKind D2H = hipMemcpyDeviceToHost;
