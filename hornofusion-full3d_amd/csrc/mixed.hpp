@@ -22,6 +22,7 @@ struct MxDyn {
 
 struct MxStat {
     double bnorm, b1, res_l2, res_l1;
+    double res_first, res_least;   // res_l2 of the first step, the smallest so far
     double mean_x[MAX_COMP];
     int n_refine, done, status, xbuf;
 };

@@ -14,7 +14,7 @@ import pytest
 
 import eafp
 import oracle
-from eafp import systems
+from eafp import _lib, systems
 
 pytestmark = pytest.mark.gpu
 
@@ -171,3 +171,34 @@ def test_fp64_default_does_not_stream():
         b.set_tiling(2, 0)
         b.solve_fp64(tol=1e-8)
         assert eafp.counters()["graph_launches"] > c0
+
+
+@pytest.mark.parametrize("shape,seed,fmt,precond", [
+    ((9, 28, 68), 1, "COEF_FP16", "PRECOND_ZLINE"),
+    ((27, 31, 34), 2, "COEF_FP16", "PRECOND_ZLINE"),
+    ((10, 85, 9), 3, "COEF_FP16", "PRECOND_JACOBI"),
+    ((16, 52, 9), 4, "COEF_FP16", "PRECOND_JACOBI"),
+])
+def test_a_solve_that_diverges_is_the_streaming_one(shape, seed, fmt, precond):
+    """16-bit weights can round a system into one that refinement does not
+    solve.  What such a solve leaves is the streaming kernels' result, bit for
+    bit; one that converges agrees with theirs to the tolerance."""
+    ps = systems.make_system(4, seed, shape)
+    print(f"case diverging shape={shape} seed={seed} {fmt} {precond}", flush=True)
+    out = []
+    for streaming in (False, True):
+        with eafp.Batch([shape]) as B:
+            if streaming:
+                i = B.info()
+                B.set_tiling(i["tile_cells"] // 256, i["grid"])
+            B.upload(0, ps)
+            st = B.solve_mixed(tol=1e-10, max_steps=600, coef_format=getattr(_lib, fmt),
+                               precond=getattr(_lib, precond))[0]
+            out.append((st, B.download(0)))
+    (a, pa), (b, pb) = out
+    print(a["status"], a["n_refine"], a["residual"], b["status"], b["n_refine"], b["residual"], flush=True)
+    assert a["status"] == b["status"]
+    if b["status"] == "converged":
+        assert np.abs(pa - pb).max() <= 1e-6 * np.abs(pb).max()
+    else:
+        assert np.array_equal(pa, pb) and a["n_iter"] == b["n_iter"]
