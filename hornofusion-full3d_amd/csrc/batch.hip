@@ -507,7 +507,11 @@ bool HostRing::open(long want) {
     if (!ok) mem = nullptr;
     for (hipEvent_t& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     none = !ok;
-    if (none) (void)hipGetLastError();
+    if (none) {
+        if (mem) (void)hipHostFree(mem);
+        mem = nullptr;
+        (void)hipGetLastError();
+    }
     return ok;
 }
 
