@@ -1639,31 +1639,39 @@ __global__ __launch_bounds__(BLOCK) void k_mreplace_line(MxArgs a) {
 
 // Finished systems, straight into the host's memory (through device memory
 // and a copy, a step of one 60x120x84 system took 8 us longer); -1
-// when a resident launch was given up, -2 from the step on in which a system
-// of a resident solve diverges.  Opens the gate of the next resident launch,
-// whose tags begin after this one's.
+// when a resident launch was given up.  Opens the gate of the next resident
+// launch, whose tags begin after this one's.
 //
 // FP16 weights (BF16 now and then) can round a system into one whose
 // corrections no longer reduce the residual; what is left after max_steps
-// then hangs on every rounding, the order of the sums included.  Such a solve
-// begins again with the streaming kernels and ends where it always did.  A
+// then hangs on every rounding, the order of the sums included.  Such a system
+// begins again with the streaming kernels and ends where it always did: here it
+// is set aside (status MX_ASIDE, counted in ndone[1]), the others go on on
+// chip, and k_mrestart takes it up once they are done.  A
 // system counts as diverging when its residual is four times the first one or
-// 64 times the least so far: over 1233 solves of drawn meshes, all 66 that did
-// not converge passed that (half of them within 16 steps of 2000), and of the
-// 1167 that did none passed 2 and 25.  A system of fewer than 512 cells is left
+// 64 times the least so far: over 19286 solves of drawn systems, all 177 that did
+// not converge passed that (half of them within 20 steps of 2000, the last
+// after 396), and so did 25 of the 19109 that did converge, which then only take the longer
+// way.  A system of fewer than 512 cells is left
 // alone: the inner CG can solve it within a step, and its residual then jumps
 // up and down with either kernel before it gets there.
 constexpr double MX_FAR_FIRST = 4.0, MX_FAR_LEAST = 64.0;
 constexpr int MX_FAR_CELLS = 512;
+constexpr int MX_ASIDE = -1;   // MxStat::status, between k_mcount and k_mrestart only
 __global__ __launch_bounds__(BLOCK) void k_mcount(MxArgs a, unsigned* gate, unsigned tags) {
     __shared__ double sh[2 * BLOCK / 64];
     double v[2] = {0.0, 0.0};
     for (int s = threadIdx.x; s < a.nsys; s += BLOCK) {
-        const MxStat& S = a.stat[1][s];
-        v[0] += S.done ? 1.0 : 0.0;
-        v[1] += S.res_l2 > fmin(MX_FAR_FIRST * S.res_first, MX_FAR_LEAST * S.res_least) && a.geom[s].n >= MX_FAR_CELLS
-                    ? 1.0
-                    : 0.0;
+        MxStat& S = a.stat[1][s];
+        int done = S.done;
+        if (gate && S.status != EAFP_STOP_CONVERGED && S.status != MX_ASIDE && a.geom[s].n >= MX_FAR_CELLS &&
+            S.res_l2 > fmin(MX_FAR_FIRST * S.res_first, MX_FAR_LEAST * S.res_least)) {
+            S.done = done = 1;
+            S.status = MX_ASIDE;
+            a.dyn[1][s].done = 1;
+        }
+        v[0] += done ? 1.0 : 0.0;
+        v[1] += done && S.status == MX_ASIDE ? 1.0 : 0.0;
     }
     block_sum<2>(v, sh);
     if (threadIdx.x == 0) {
@@ -1674,12 +1682,19 @@ __global__ __launch_bounds__(BLOCK) void k_mcount(MxArgs a, unsigned* gate, unsi
             } else {
                 gate[0] = 0;
                 gate[1] += tags;
-                if (v[1] > 0.0) gate[2] = 1;
-                if (gate[2]) n = -2;
             }
         }
+        __hip_atomic_store(a.ndone + 1, (int)v[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         __hip_atomic_store(a.ndone, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+}
+
+// The systems set aside begin again; the others stay done.
+__global__ __launch_bounds__(BLOCK) void k_mrestart(MxArgs a) {
+    const int s = blockIdx.x * BLOCK + threadIdx.x;
+    if (s >= a.nsys || a.stat[1][s].status != MX_ASIDE) return;
+    a.stat[1][s] = MxStat{};
+    a.dyn[1][s] = MxDyn{};
 }
 
 // ---------------------------------------------------------------------------
@@ -1721,7 +1736,7 @@ struct MixedWork {
     DevBuf<MxDyn> dyn0, dyn1;
     DevBuf<MxStat> stat0, stat1;
     DevBuf<MxConst> cst;
-    int* host_cnt = nullptr;        // pinned: k_mcount's result
+    int* host_cnt = nullptr;        // pinned: k_mcount's two results
     hipEvent_t ev[2] = {nullptr, nullptr};
     hipEvent_t t0 = nullptr, t1 = nullptr;
     GraphCache<MxArgs> graphs;      // one instantiated graph per (format, interval, precond, shape, buffers)
@@ -1802,7 +1817,7 @@ static int init_mixed(Batch& B, MixedWork* w) {
         EAFP_TRY_RC(w->stat0.alloc(B.nsys));
         EAFP_TRY_RC(w->stat1.alloc(B.nsys));
         EAFP_TRY_RC(w->cst.alloc(B.nsys));
-        EAFP_TRY(hipHostMalloc((void**)&w->host_cnt, sizeof(int), hipHostMallocDefault));
+        EAFP_TRY(hipHostMalloc((void**)&w->host_cnt, 2 * sizeof(int), hipHostMallocDefault));
         for (auto& e : w->ev) EAFP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         EAFP_TRY(hipEventCreate(&w->t0));
         EAFP_TRY(hipEventCreate(&w->t1));
@@ -2075,18 +2090,31 @@ static int check_mixed(Batch& B, const eafp_mixed_opts& o) {
     return EAFP_OK;
 }
 
-// Setup and the refinement steps until every system is finished.  *again < 0:
-// the solve has to begin again, streaming: a resident launch did not get its
-// CUs (-1, resident.hpp) or a system diverges (-2, k_mcount).  Returns with the stream idle but for the launch after the
+// The refinement steps until every system is finished: of all systems, or
+// (MX_SET_ASIDE) of those that a resident solve has set aside.  *given_up: a
+// resident launch did not get its CUs (resident.hpp), the solve has to begin
+// again, streaming.  *aside: systems that a resident solve has set aside
+// (k_mcount).  Returns with the stream idle but for the launch after the
 // last one needed.
-static int mixed_steps(Batch& B, const eafp_mixed_opts& o, int fmt, int interval, bool resident, int* again) {
+enum { MX_STREAM, MX_RESIDENT, MX_SET_ASIDE };
+static int mixed_steps(Batch& B, const eafp_mixed_opts& o, int fmt, int interval, int mode, bool* given_up,
+                       int* aside) {
     MixedWork* w = B.mixed;
-    *again = 0;
+    const bool resident = mode == MX_RESIDENT;
+    *given_up = false;
+    *aside = 0;
     EAFP_TRY_RC(mixed_graph(B, fmt, interval, resident));
     const long max_launch = (long)o.max_steps + 2;
     const long tags = resident ? resident_tags(*w->res, interval) : 0;
     if (resident) EAFP_TRY_RC(w->res->arm(0, B.stream));
-    EAFP_TRY_RC(mixed_start(B, o, fmt));
+    if (mode == MX_SET_ASIDE) {
+        // the weights, their factors and the options are in place
+        k_mrestart<<<(B.nsys + BLOCK - 1) / BLOCK, BLOCK, 0, B.stream>>>(w->args);
+        launch_refine(B);
+        EAFP_TRY(hipGetLastError());
+    } else {
+        EAFP_TRY_RC(mixed_start(B, o, fmt));
+    }
 
     // One graph launch = one refinement step for every system; poll the
     // finished count behind the step before the one just launched (or that
@@ -2103,7 +2131,7 @@ static int mixed_steps(Batch& B, const eafp_mixed_opts& o, int fmt, int interval
             if (resident && w->res->tag > 0xF0000000u - 2 * (unsigned)tags) {   // begin the tags again
                 EAFP_TRY(hipStreamSynchronize(B.stream));
                 if (finished() < 0) {
-                    *again = finished();
+                    *given_up = true;
                     return EAFP_OK;
                 }
                 EAFP_TRY_RC(w->res->arm(0x20000000, B.stream));
@@ -2122,7 +2150,8 @@ static int mixed_steps(Batch& B, const eafp_mixed_opts& o, int fmt, int interval
     }
     if (resident) {
         EAFP_TRY(hipStreamSynchronize(B.stream));   // the CUs are free again
-        *again = std::min(finished(), 0);
+        *given_up = finished() < 0;
+        *aside = w->host_cnt[1];
     }
     return EAFP_OK;
 }
@@ -2136,18 +2165,18 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
     int interval = o.interval > 0 ? o.interval : 32;
     interval = (interval + 1) & ~1;    // even: the p buffer parity restarts every step
     EAFP_TRY(hipEventRecord(w->t0, B.stream));
-    int again = 0;
+    bool given_up = true;
+    int aside = 0;
     // a step's tags have to fit the 32 bits several times over (resident.hpp);
     // longer steps, of millions of iterations, stream
     if (B.resident_mixed && w->res && !w->res->given_up && resident_tags(*w->res, interval) < RES_STEP_TAGS) {
         const ResPlan& p = w->res->plan;
         const ResidentGate held(p.members);
-        EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, true, &again));
-        w->res->given_up = again == -1;
-    } else {
-        again = 1;
+        EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, MX_RESIDENT, &given_up, &aside));
+        w->res->given_up = given_up;
     }
-    if (again) EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, false, &again));
+    if (given_up) EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, MX_STREAM, &given_up, &aside));
+    else if (aside) EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, MX_SET_ASIDE, &given_up, &aside));
     k_mproject<<<B.grid, BLOCK, 0, B.stream>>>(w->args, BLOCK * B.cpt);
     EAFP_TRY(hipGetLastError());
     EAFP_TRY_RC(download_all(B, w->xout.p));

@@ -68,7 +68,7 @@ struct MxArgs {
     MxDyn* dyn[2];
     MxStat* stat[2];
     const MxConst* cst;
-    int* ndone;
+    int* ndone;          // finished systems; of them, set aside (k_mcount)
 };
 
 // ---------------------------------------------------------------------------

@@ -78,8 +78,7 @@ struct ResLaunch {
     const int2* member;
     int nteam, T;
     u64* slots;         // 2 * T * SLOT_WORDS of every team
-    unsigned* gate;     // [0] arrivals and the give-up mark, [1] the next launch's first tag,
-                        // [2] a mark of the solver's own
+    unsigned* gate;     // [0] arrivals and the give-up mark, [1] the next launch's first tag
     int expected;       // work-groups that pass the gate
     int pad_;
 };

@@ -232,7 +232,7 @@ int ResDevice::init(ResPlan&& p, hipStream_t stream) {
     EAFP_TRY_RC(items.alloc(p.items.size()));
     EAFP_TRY_RC(team_begin.alloc(p.team_begin.size()));
     EAFP_TRY_RC(slots.alloc((size_t)p.nslot * SLOT_WORDS));
-    EAFP_TRY_RC(gate.alloc(3));
+    EAFP_TRY_RC(gate.alloc(2));
     EAFP_TRY(hipMemcpy(items.p, p.items.data(), sizeof(ResItem) * p.items.size(), hipMemcpyHostToDevice));
     EAFP_TRY(hipMemcpy(team_begin.p, p.team_begin.data(), sizeof(int) * p.team_begin.size(), hipMemcpyHostToDevice));
     if (!p.T) {
@@ -242,7 +242,7 @@ int ResDevice::init(ResPlan&& p, hipStream_t stream) {
         EAFP_TRY(hipMemcpy(member.p, p.member.data(), sizeof(int2) * p.member.size(), hipMemcpyHostToDevice));
     }
     EAFP_TRY(hipMemsetAsync(slots.p, 0, sizeof(u64) * slots.n, stream));
-    EAFP_TRY(hipMemsetAsync(gate.p, 0, sizeof(unsigned) * 3, stream));
+    EAFP_TRY(hipMemsetAsync(gate.p, 0, sizeof(unsigned) * 2, stream));
     tag = 1;
     plan = std::move(p);
     return EAFP_OK;
@@ -265,7 +265,6 @@ ResLaunch ResDevice::launch() const {
 __global__ void k_res_arm(unsigned* gate, unsigned tag) {
     gate[0] = 0;
     gate[1] = tag;
-    gate[2] = 0;
 }
 
 int ResDevice::take_tags(long tags, hipStream_t stream, unsigned* first) {
