@@ -46,14 +46,13 @@ struct Cg64Work {
     hipGraphExec_t exec = nullptr;  // the cached graph of the current solve
     Cg64Args args{};
     std::unique_ptr<ResDevice> res;  // resident solve, when the batch fits on chip
-    DevBuf<double> zx;               // its exchange buffer
     CgSlot* slots_host = nullptr;    // pinned: the slots after a resident launch
     unsigned* gate_host = nullptr;   // pinned: its gate word
 };
 
 ResPlan plan_resident64(const Batch& B);
 int start_resident64(Batch& B, ResDevice& D, CgSlot* slot, CgConst* cst, double tol, int max_iter, int iters);
-int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int iters, bool first);
+int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, int iters, bool first);
 int report_resident64(Batch& B, ResDevice& D, const CgSlot* slot, CgSlot* slots_host, unsigned* gate_host);
 
 void free_cg64(Cg64Work* w) {
@@ -372,12 +371,19 @@ static int init_cg64(Batch& B, Cg64Work* w) {
         EAFP_TRY(hipMemset(w->p0.p, 0, n * sizeof(double)));
         EAFP_TRY(hipMemset(w->p1.p, 0, n * sizeof(double)));
         ResPlan plan = plan_resident64(B);
-        EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, w->zx, B.stream));
+        EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, B.stream));
         if (w->res) {
             EAFP_TRY(hipHostMalloc((void**)&w->slots_host, sizeof(CgSlot) * B.nsys, hipHostMallocDefault));
             EAFP_TRY(hipHostMalloc((void**)&w->gate_host, sizeof(unsigned), hipHostMallocDefault));
         }
     }
+    return EAFP_OK;
+}
+
+// The buffers that hang on the launch shape.
+static int size_cg64(Batch& B, Cg64Work* w) {
+    EAFP_TRY_RC(w->partA.alloc((size_t)B.ntiles));
+    EAFP_TRY_RC(w->partB.alloc((size_t)B.ntiles * 3));
     return EAFP_OK;
 }
 
@@ -392,8 +398,14 @@ static int ensure_cg64(Batch& B) {
         B.cg64 = nw;
     }
     Cg64Work* w = B.cg64;
-    EAFP_TRY_RC(w->partA.alloc((size_t)B.ntiles));
-    EAFP_TRY_RC(w->partB.alloc((size_t)B.ntiles * 3));
+    int rc = size_cg64(B, w);
+    if (rc == (int)hipErrorOutOfMemory && w->res) {   // without the resident form, then
+        (void)hipGetLastError();
+        EAFP_TRY(hipStreamSynchronize(B.stream));
+        w->res.reset();
+        rc = size_cg64(B, w);
+    }
+    EAFP_TRY_RC(rc);
     Cg64Args& a = w->args;
     a.tiles = B.tiles.p;
     a.ntiles = B.ntiles;
@@ -507,7 +519,7 @@ static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* s
     EAFP_TRY_RC(start_resident64(B, D, w->slot1.p, w->cst.p, tol, max_iter, RES_ITERS));
     const ResidentGate held(D.plan.members);
     for (bool first = true;; first = false) {
-        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, RES_ITERS, first));
+        EAFP_TRY_RC(launch_resident64(B, D, w->args, RES_ITERS, first));
         EAFP_TRY_RC(download_all(B, w->x.p));
         EAFP_TRY(hipEventRecord(w->t1, B.stream));
         EAFP_TRY_RC(report_resident64(B, D, w->slot1.p, w->slots_host, w->gate_host));
@@ -598,7 +610,7 @@ int time_resident64(Batch& B, int iters, float* ms) {
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
         EAFP_TRY_RC(start_resident64(B, D, w->slot1.p, w->cst.p, 0.0, 1 << 30, iters));
         EAFP_TRY(hipEventRecord(w->t0, B.stream));
-        EAFP_TRY_RC(launch_resident64(B, D, w->args, w->zx.p, iters, true));
+        EAFP_TRY_RC(launch_resident64(B, D, w->args, iters, true));
         EAFP_TRY(hipEventRecord(w->t1, B.stream));
         EAFP_TRY_RC(report_resident64(B, D, w->slot1.p, w->slots_host, w->gate_host));
         EAFP_TRY(hipStreamSynchronize(B.stream));

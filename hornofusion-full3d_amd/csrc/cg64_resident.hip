@@ -31,7 +31,8 @@ namespace eafp {
 struct R64Args {
     Cg64Args a;
     ResLaunch L;
-    double* zx;          // exchange buffer, ResItem::xoff + row * nz + k
+    double* zx;          // edge rows of z for the neighbours, ResItem::xoff + row * nz + k: the
+                         // streaming kernels' q, which has the same places and is free here
     int iters;           // iterations per item and launch at most
 };
 
@@ -399,13 +400,13 @@ int report_resident64(Batch& B, ResDevice& D, const CgSlot* slot, CgSlot* slots_
 // One launch: at most `iters` iterations of every unfinished system.  The
 // slots, x0, b, fold and the coefficients are the streaming kernels' own.
 // `first`: start_resident64 has opened the gate.
-int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, double* zx, int iters, bool first) {
+int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, int iters, bool first) {
     const ResPlan& p = D.plan;
     if (!first) EAFP_TRY_RC(D.arm(launch_tags(D, iters), B.stream));
     R64Args g{};
     g.a = a;
     g.L = D.launch();
-    g.zx = zx;
+    g.zx = a.q;
     g.iters = iters;
     const size_t lds = std::max(p.lds, p.members > 0 ? (size_t)RES_LDS_ALONE : (size_t)0);
     switch (p.slots) {

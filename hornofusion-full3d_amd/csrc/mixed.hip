@@ -1748,7 +1748,7 @@ struct MixedWork {
     MxArgs args{};
     std::unique_ptr<ResDevice> res; // resident inner iterations, when the batch fits on chip
     int res_cq = 1;                 // quads per lane
-    DevBuf<float> xz;               // their exchange buffer
+    DevBuf<float> xz;               // their exchange buffer, where r64 is too small for it
 };
 
 void free_mixed(MixedWork* w) {
@@ -1796,6 +1796,25 @@ static ResPlan plan_resident_mixed(const Batch& B, int* cq) {
     return *cq == 2 ? std::move(p2) : std::move(p1);
 }
 
+// The resident form, where the batch has one.  The neighbours' rows are
+// exchanged through r64, which the inner iterations leave alone (8 bytes per
+// cell; a row takes 4 per cell, rounded up to whole lanes: only rows of 1 to 3
+// cells may need more).
+static int plan_mixed(Batch& B, MixedWork* w) {
+    ResPlan plan = plan_resident_mixed(B, &w->res_cq);
+    const long xlen = plan.xlen;
+    EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, B.stream));
+    if (w->res && xlen > 2 * B.ncells) {
+        const int rc = w->xz.alloc(xlen);
+        if (rc != EAFP_OK) {
+            w->res.reset();
+            if (rc != (int)hipErrorOutOfMemory) return rc;
+            (void)hipGetLastError();
+        }
+    }
+    return EAFP_OK;
+}
+
 // First-time buffers of the mixed solver; the caller publishes w only when
 // every one of them exists.
 static int init_mixed(Batch& B, MixedWork* w) {
@@ -1825,23 +1844,13 @@ static int init_mixed(Batch& B, MixedWork* w) {
         for (auto& e : w->ev) EAFP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         EAFP_TRY(hipEventCreate(&w->t0));
         EAFP_TRY(hipEventCreate(&w->t1));
-        ResPlan plan = plan_resident_mixed(B, &w->res_cq);
-        EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, w->xz, B.stream));
+        EAFP_TRY_RC(plan_mixed(B, w));
     }
     return EAFP_OK;
 }
 
-static int ensure_mixed(Batch& B, int fmt) {
-    if (!B.mixed) {
-        MixedWork* nw = new MixedWork();
-        const int rc = init_mixed(B, nw);
-        if (rc != EAFP_OK) {
-            free_mixed(nw);
-            return rc;
-        }
-        B.mixed = nw;
-    }
-    MixedWork* w = B.mixed;
+// The buffers that hang on the format, the launch shape or the line tiles.
+static int size_mixed(Batch& B, MixedWork* w, int fmt) {
     if (w->fmt != fmt) {
         const size_t n = B.ncells;
         w->fmt = -1;   // a failed allocation below leaves the weights invalid, not stale
@@ -1868,6 +1877,30 @@ static int ensure_mixed(Batch& B, int fmt) {
         EAFP_TRY_RC(w->fac.alloc(B.ncells + SINK_CELLS));
         EAFP_TRY(hipMemsetAsync(w->fac.p, 0, (B.ncells + SINK_CELLS) * sizeof(unsigned), B.stream));
     }
+    return EAFP_OK;
+}
+
+static int ensure_mixed(Batch& B, int fmt) {
+    if (!B.mixed) {
+        MixedWork* nw = new MixedWork();
+        const int rc = init_mixed(B, nw);
+        if (rc != EAFP_OK) {
+            free_mixed(nw);
+            return rc;
+        }
+        B.mixed = nw;
+    }
+    MixedWork* w = B.mixed;
+    int rc = size_mixed(B, w, fmt);
+    if (rc == (int)hipErrorOutOfMemory && w->res) {   // without the resident form, then
+        (void)hipGetLastError();
+        EAFP_TRY(hipStreamSynchronize(B.stream));
+        w->graphs.clear();
+        w->res.reset();
+        w->xz.release();
+        rc = size_mixed(B, w, fmt);
+    }
+    EAFP_TRY_RC(rc);
     MxArgs& a = w->args;
     a.tiles = B.tiles.p;
     a.ntiles = B.ntiles;
@@ -1996,7 +2029,7 @@ static int launch_resident_mixed(Batch& B, int fmt, int interval) {
     RMxArgs g{};
     g.a = w->args;
     g.L = w->res->launch();
-    g.xz = w->xz.p;
+    g.xz = w->xz.p ? w->xz.p : reinterpret_cast<float*>(w->r64.p);
     g.interval = interval;
     const size_t lds = std::max(p.lds, p.members > 0 ? (size_t)RES_LDS_ALONE : (size_t)0);
     const bool line = w->args.line != 0;

@@ -248,6 +248,16 @@ int ResDevice::init(ResPlan&& p, hipStream_t stream) {
     return EAFP_OK;
 }
 
+int ResDevice::create(ResPlan&& p, std::unique_ptr<ResDevice>& out, hipStream_t stream) {
+    if (!p.ok) return EAFP_OK;
+    auto d = std::make_unique<ResDevice>();
+    const int rc = d->init(std::move(p), stream);
+    if (rc == EAFP_OK) out = std::move(d);
+    if (rc != (int)hipErrorOutOfMemory) return rc;
+    (void)hipGetLastError();
+    return EAFP_OK;
+}
+
 ResLaunch ResDevice::launch() const {
     ResLaunch L{};
     L.items = items.p;

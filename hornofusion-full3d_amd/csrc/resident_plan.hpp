@@ -55,7 +55,9 @@ class ResidentGate {
     int dev_, n_;
 };
 
-// A plan's tables on the device.
+// A plan's tables on the device: some kilobytes, as rows are exchanged through an
+// array that the solver's resident kernel does not use otherwise, and given
+// back should the solver run out of memory later.
 struct ResDevice {
     ResPlan plan;
     DevBuf<ResItem> items;
@@ -68,23 +70,9 @@ struct ResDevice {
     bool given_up = false;        // a launch did not get its CUs: stream from now on
     int init(ResPlan&& p, hipStream_t stream);
     ResLaunch launch() const;
-    // `out` and its exchange buffer; both stay empty, and the batch streams,
-    // where the plan is not ok or the device's memory does not hold them
-    template <typename X>
-    static int create(ResPlan&& p, std::unique_ptr<ResDevice>& out, DevBuf<X>& exchange, hipStream_t stream) {
-        if (!p.ok) return EAFP_OK;
-        auto d = std::make_unique<ResDevice>();
-        int rc = exchange.alloc(p.xlen);
-        if (rc == EAFP_OK) rc = d->init(std::move(p), stream);
-        if (rc == EAFP_OK) {
-            out = std::move(d);
-            return EAFP_OK;
-        }
-        exchange.release();
-        if (rc != (int)hipErrorOutOfMemory) return rc;
-        (void)hipGetLastError();
-        return EAFP_OK;
-    }
+    // `out` stays empty, and the batch streams, where the plan is not ok or the
+    // device's memory does not hold its tables
+    static int create(ResPlan&& p, std::unique_ptr<ResDevice>& out, hipStream_t stream);
     // gate open and `tag` set for the next launch, which uses at most `tags` of them
     int arm(long tags, hipStream_t stream);
     // the first of `tags` tags, for a kernel that opens the gate itself
