@@ -594,6 +594,8 @@ struct PPWork {
     DevBuf<int> ct, outlet, masks, lki;
     DevBuf<unsigned char> act;       // k_pp_act's bytes
     double* part_h = nullptr;        // pinned: the blocks' sums, which the kernel stores there itself
+    DevBuf<double> part;             // where there is no pinned memory: the sums on the device,
+    std::vector<double> part_v;      // and copied
     ~PPWork() {
         if (part_h) (void)hipHostFree(part_h);
     }
@@ -624,7 +626,10 @@ int ensure_pp(const eafp_desc* d) {
     const long blocks = pp_blocks(n, (long)(d->nr + 4) * (d->ntheta + 4));
     if (w.part_h) (void)hipHostFree(w.part_h);
     w.part_h = nullptr;
-    EAFP_TRY(hipHostMalloc((void**)&w.part_h, sizeof(double) * 2 * blocks, hipHostMallocDefault));
+    if (!pinned_alloc(&w.part_h, (size_t)blocks * 2)) {
+        EAFP_TRY_RC(w.part.alloc((size_t)blocks * 2));
+        w.part_v.assign((size_t)blocks * 2, 0.0);
+    }
     w.nr = d->nr;
     w.nth = d->ntheta;
     w.nz = d->nz;
@@ -784,7 +789,8 @@ int pp_assemble(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_confi
     a.gz = w.grads.p + 2 * n;
     a.gzg = w.grads.p + 3 * n;
     a.act = w.act.p;
-    EAFP_TRY(hipHostGetDevicePointer((void**)&a.part, w.part_h, 0));
+    a.part = w.part.p;
+    if (w.part_h) EAFP_TRY(hipHostGetDevicePointer((void**)&a.part, w.part_h, 0));
     const int blocks = pp_blocks(n, a.sz);
     k_pp_act<<<blocks, BLOCK, 0, w.stream>>>(a);
     k_pp_grad<<<blocks, BLOCK, 0, w.stream>>>(a);
@@ -801,11 +807,14 @@ int pp_assemble(const eafp_desc* d, const eafp_pp_fields* f, const eafp_pp_confi
                 EAFP_TRY(hipMemcpyAsync(ex_i[q], w.lki.p + (long)q * n, sizeof(int) * n, D2H, w.stream));
         }
     }
+    if (!w.part_h)
+        EAFP_TRY(hipMemcpyAsync(w.part_v.data(), w.part.p, sizeof(double) * 2 * blocks, hipMemcpyDeviceToHost, w.stream));
     EAFP_TRY(hipStreamSynchronize(w.stream));
+    const double* part = w.part_h ? w.part_h : w.part_v.data();
     double fl = 0.0, su = 0.0;
     for (int b = 0; b < blocks; ++b) {
-        fl += w.part_h[2 * (size_t)b];
-        su += w.part_h[2 * (size_t)b + 1];
+        fl += part[2 * (size_t)b];
+        su += part[2 * (size_t)b + 1];
     }
     if (flux_ref) *flux_ref = fl;
     if (residual) *residual = su / std::max(fl, SMALL);

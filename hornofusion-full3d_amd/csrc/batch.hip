@@ -503,8 +503,7 @@ int Batch::label_components() {
 bool HostRing::open(long want) {
     if (mem || none) return mem != nullptr;
     len = std::min(want, SLOT_LEN);
-    bool ok = hipHostMalloc((void**)&mem, sizeof(double) * len * SLOTS, hipHostMallocDefault) == hipSuccess;
-    if (!ok) mem = nullptr;
+    bool ok = pinned_alloc(&mem, (size_t)len * SLOTS);
     for (hipEvent_t& e : ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
     none = !ok;
     if (none) {

@@ -55,6 +55,15 @@ struct DevBuf {
     }
 };
 
+// Pinned host memory that its caller can do without; false: there is none.
+template <typename T>
+bool pinned_alloc(T** p, size_t n) {
+    if (hipHostMalloc((void**)p, sizeof(T) * n, hipHostMallocDefault) == hipSuccess) return true;
+    *p = nullptr;
+    (void)hipGetLastError();
+    return false;
+}
+
 // Instantiated graphs of one solver, kept until the solver's workspace is
 // freed.  An entry's key is the solver's integer settings (format,
 // preconditioner, iterations per graph, launch-shape generation) together

@@ -372,10 +372,8 @@ static int init_cg64(Batch& B, Cg64Work* w) {
         EAFP_TRY(hipMemset(w->p1.p, 0, n * sizeof(double)));
         ResPlan plan = plan_resident64(B);
         EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, B.stream));
-        if (w->res) {
-            EAFP_TRY(hipHostMalloc((void**)&w->slots_host, sizeof(CgSlot) * B.nsys, hipHostMallocDefault));
-            EAFP_TRY(hipHostMalloc((void**)&w->gate_host, sizeof(unsigned), hipHostMallocDefault));
-        }
+        if (w->res && !(pinned_alloc(&w->slots_host, B.nsys) && pinned_alloc(&w->gate_host, 1)))
+            w->res.reset();   // nowhere to report to: the streaming kernels
     }
     return EAFP_OK;
 }

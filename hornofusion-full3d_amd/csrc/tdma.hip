@@ -380,15 +380,12 @@ bool overlap_pays(int nsys, const eafp_desc* d) {
     return nsys <= TD_OVERLAP_SYS && steps >= TD_OVERLAP_STEPS;
 }
 
-// off_h for n flags.
-int ensure_flags(TdWork& w, size_t n) {
-    if (w.off_n >= n) return EAFP_OK;
+// off_h for n flags; false: there is no pinned memory.
+bool ensure_flags(TdWork& w, size_t n) {
+    if (w.off_n >= n) return true;
     if (w.off_h) (void)hipHostFree(w.off_h);
-    w.off_h = nullptr;
-    w.off_n = 0;
-    EAFP_TRY(hipHostMalloc((void**)&w.off_h, sizeof(int) * n, hipHostMallocDefault));
-    w.off_n = n;
-    return EAFP_OK;
+    w.off_n = pinned_alloc(&w.off_h, n) ? n : 0;
+    return w.off_n > 0;
 }
 
 int halo_lines(int P, int nu, int nv) { return P == 0 ? 2 * nu + nv : P == 1 ? 2 * nv + 2 * nu : 2 * nv + nu; }
@@ -530,9 +527,8 @@ int tdma_solve_batch(int nsys, const eafp_desc* descs, const eafp_tdma_system* s
     k_tdma_setup<<<g_lines, TD_BLOCK, 0, w.stream>>>(tp);
     // Overlapped sweeps, where every pass of every system runs the chain kernel,
     // which the setup decides last
-    bool overlap = chain[0] && chain[1] && chain[2] && overlap_pays(nsys, descs);
+    bool overlap = chain[0] && chain[1] && chain[2] && overlap_pays(nsys, descs) && ensure_flags(w, 3 * (size_t)nsys);
     if (overlap) {
-        EAFP_TRY_RC(ensure_flags(w, 3 * (size_t)nsys));
         EAFP_TRY(hipMemcpyAsync(w.off_h, icur, sizeof(int) * 3 * nsys, hipMemcpyDeviceToHost, w.stream));
         EAFP_TRY(hipStreamSynchronize(w.stream));
         for (int q = 0; q < 3 * nsys; ++q) overlap = overlap && !w.off_h[q];

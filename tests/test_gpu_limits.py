@@ -52,3 +52,50 @@ for kind in ("fp64", "mixed"):
 
 def test_what_a_solve_can_do_without_costs_no_other_piece(tmp_path):
     limits.run(tmp_path, DEVICE)
+
+
+PINNED = '''
+ps = systems.make_system(2, 0, (20, 30, 33))
+mesh = eafp.Mesh(*ps.shape)
+F, cfg = fields.make_fields(*ps.shape, seed=3, masks=True)
+tm = (35, 66, 49)                # large enough for overlapped passes
+tps = systems.make_system(3, 0, tm)
+names = ("aW", "aE", "aS", "aN", "aB", "aT", "aP", "Su")
+
+def passes():
+    coef = [np.array(ps.padded(n), order="F") for n in names]
+    phi = np.zeros_like(coef[0], order="F")
+    res, nit = eafp.cg_3d_mpi(*coef, phi, mesh, 30, 1e-30)
+    out = {"cg": phi}
+    assert nit == 30
+    with eafp.Batch.from_systems([ps]) as b:
+        st = b.solve_fp64(30, 1e-30)
+        out["fp64"] = b.download(0)
+        assert st[0]["n_iter"] == 30
+        st = b.solve_mixed(tol=1e-10)
+        assert st[0]["status"] == "converged"
+        out["mixed"] = b.download(0)
+    coef, res, flux = eafp.pp_assemble(F, cfg, mesh)
+    out.update(coef, residual=np.array([res, flux]))
+    t = [np.array(tps.padded(n), order="F") for n in names]
+    f = np.asfortranarray(np.random.default_rng(1).normal(size=t[0].shape))
+    eafp.tdma_3d_mpi(*t, f, eafp.Mesh(*tm), 2)
+    out["tdma"] = f
+    eafp.release()
+    return out
+
+with_it = passes()
+shim.shim_pinned(8)              # the solvers' two counters, and nothing else
+without = passes()
+print("case", sorted(with_it), flush=True)
+for n in with_it:
+    if n in ("cg", "fp64", "mixed"):     # streaming instead of resident: the sums have another order
+        tol = 1e-6 if n == "mixed" else 1e-12
+        assert np.abs(with_it[n] - without[n]).max() <= tol * np.abs(with_it[n]).max(), n
+    else:
+        assert np.array_equal(with_it[n], without[n], equal_nan=True), n
+'''
+
+
+def test_without_pinned_memory(tmp_path):
+    limits.run(tmp_path, PINNED)
