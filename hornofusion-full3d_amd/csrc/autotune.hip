@@ -72,16 +72,16 @@ int autotune(Batch& B, int solver, int fmt, int reps, int* best_cpt, int* best_b
         EAFP_TRY_RC(B.set_columns(bs));
         float ms = 0.f;
         EAFP_TRY_RC(time_resident_mixed(B, fmt, solver == 2 ? EAFP_PRECOND_ZLINE : EAFP_PRECOND_JACOBI, 32, &ms));
-        B.resident_mixed = ms > 0.f && ms < best;
-        if (B.resident_mixed) best = ms;
+        if (ms > 0.f) B.resident_mixed = ms < best;   // not timed: as it was
+        if (ms > 0.f && ms < best) best = ms;
     }
     // the systems on chip, where they fit: kept when that is faster than the
     // best streaming shape
     if (solver == 0) {
         float ms = 0.f;
         EAFP_TRY_RC(time_resident64(B, 16 * reps, &ms));
-        B.resident64 = ms > 0.f && ms < best;
-        if (B.resident64) best = ms;
+        if (ms > 0.f) B.resident64 = ms < best;
+        if (ms > 0.f && ms < best) best = ms;
     }
     if (best_cpt) *best_cpt = bc;
     if (best_blocks) *best_blocks = bb;

@@ -6,10 +6,13 @@
 #include <mutex>
 
 #include "batch.hpp"
+#include "resident_plan.hpp"
 
 namespace eafp {
 int solve_fp64(Batch& B, int max_iter, double tol, eafp_stats* stats, int chunk);
 int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats);
+ResDevice* resident_fp64(const Batch& B);
+ResDevice* resident_mixed(const Batch& B);
 int time_kernels(Batch& B, int solver, int fmt, int reps, float* ms_spmv, float* ms_update);
 int autotune(Batch& B, int solver, int fmt, int reps, int* best_cpt, int* best_blocks, float* best_ms);
 
@@ -221,6 +224,45 @@ int eafp_batch_components(eafp_batch* b, int s, int* nsingular, int cells[4]) {
     if (cells)
         for (int q = 0; q < eafp::MAX_COMP; ++q) cells[q] = q < c.ncomp ? c.cells[q] : 0;
     return EAFP_OK;
+}
+
+static eafp::ResDevice* resident_of(const eafp_batch* b, int solver) {
+    return solver == 0 ? eafp::resident_fp64(b->B) : eafp::resident_mixed(b->B);
+}
+
+int eafp_batch_resident(const eafp_batch* b, int solver, eafp_resident* out) {
+    if (!b || !out || solver < 0 || solver > 2) return EAFP_ERR_ARG;
+    *out = eafp_resident{};
+    const eafp::ResDevice* D = resident_of(b, solver);
+    if (!D) return EAFP_OK;
+    out->work_groups = D->plan.blocks;
+    out->teams = D->plan.nteam;
+    out->team_size = D->plan.T;
+    out->in_use = (solver == 0 ? b->B.resident64 : b->B.resident_mixed) && D->usable();
+    out->launches = D->launches;
+    out->given_up = D->given_up;
+    out->set_aside = D->aside;
+    return EAFP_OK;
+}
+
+int eafp_batch_disturb(eafp_batch* b, int solver, int what, unsigned value) {
+    if (!b || solver < 0 || solver > 2) return EAFP_ERR_ARG;
+    eafp::ResDevice* D = resident_of(b, solver);
+    if (!D) return EAFP_ERR_STATE;
+    switch (what) {
+        case EAFP_DISTURB_ABSENT:
+            if (value > 1024) return EAFP_ERR_ARG;
+            D->absent = (int)value;
+            return EAFP_OK;
+        case EAFP_DISTURB_TAG:
+            if (value < D->tag || value > 0xF0000000u) return EAFP_ERR_ARG;
+            D->tag = value;
+            return EAFP_OK;
+        case EAFP_DISTURB_PAUSE:
+            D->retry = std::chrono::steady_clock::now() + std::chrono::seconds(value);
+            return EAFP_OK;
+    }
+    return EAFP_ERR_ARG;
 }
 
 int eafp_batch_destroy(eafp_batch* b) {

@@ -516,6 +516,7 @@ static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* s
     EAFP_TRY(hipEventRecord(w->t0, B.stream));
     EAFP_TRY_RC(start_resident64(B, D, w->slot1.p, w->cst.p, tol, max_iter, RES_ITERS));
     const ResidentGate held(D.plan.members);
+    const auto since = std::chrono::steady_clock::now();
     for (bool first = true;; first = false) {
         EAFP_TRY_RC(launch_resident64(B, D, w->args, RES_ITERS, first));
         EAFP_TRY_RC(download_all(B, w->x.p));
@@ -523,7 +524,7 @@ static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* s
         EAFP_TRY_RC(report_resident64(B, D, w->slot1.p, w->slots_host, w->gate_host));
         EAFP_TRY(hipStreamSynchronize(B.stream));
         if (*w->gate_host & GATE_GIVEN_UP) {
-            D.given_up = true;
+            D.gave_up(since);
             return EAFP_OK;
         }
         bool all = true;
@@ -539,7 +540,7 @@ int solve_fp64(Batch& B, int max_iter, double tol, eafp_stats* stats, int chunk)
         if (!B.uploaded[s]) return EAFP_ERR_STATE;
     EAFP_TRY_RC(ensure_cg64(B));
     Cg64Work* w = B.cg64;
-    if (B.resident64 && w->res && !w->res->given_up) {
+    if (B.resident64 && w->res && w->res->usable()) {
         int done = 0;
         EAFP_TRY_RC(solve_fp64_resident(B, max_iter, tol, stats, &done));
         if (done) return EAFP_OK;
@@ -601,9 +602,10 @@ int time_resident64(Batch& B, int iters, float* ms) {
         if (!B.uploaded[s]) return EAFP_ERR_STATE;
     EAFP_TRY_RC(ensure_cg64(B));
     Cg64Work* w = B.cg64;
-    if (!w->res || w->res->given_up) return EAFP_OK;
+    if (!w->res || !w->res->usable()) return EAFP_OK;
     ResDevice& D = *w->res;
     const ResidentGate held(D.plan.members);
+    const auto since = std::chrono::steady_clock::now();
     iters = std::min(iters, RES_ITERS);
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
         EAFP_TRY_RC(start_resident64(B, D, w->slot1.p, w->cst.p, 0.0, 1 << 30, iters));
@@ -614,7 +616,7 @@ int time_resident64(Batch& B, int iters, float* ms) {
         EAFP_TRY(hipStreamSynchronize(B.stream));
     }
     if (*w->gate_host & GATE_GIVEN_UP) {
-        D.given_up = true;
+        D.gave_up(since);
         return EAFP_OK;
     }
     int n = 1;
@@ -663,5 +665,7 @@ int time_fp64_kernels(Batch& B, int reps, float* ms_spmv, float* ms_update) {
     if (ms_update) *ms_update = tot_u / (float)reps;
     return EAFP_OK;
 }
+
+ResDevice* resident_fp64(const Batch& B) { return B.cg64 ? B.cg64->res.get() : nullptr; }
 
 }  // namespace eafp

@@ -402,6 +402,7 @@ int report_resident64(Batch& B, ResDevice& D, const CgSlot* slot, CgSlot* slots_
 // `first`: start_resident64 has opened the gate.
 int launch_resident64(Batch& B, ResDevice& D, const Cg64Args& a, int iters, bool first) {
     const ResPlan& p = D.plan;
+    ++D.launches;
     if (!first) EAFP_TRY_RC(D.arm(launch_tags(D, iters), B.stream));
     R64Args g{};
     g.a = a;

@@ -2043,7 +2043,7 @@ static int launch_resident_mixed(Batch& B, int fmt, int interval) {
 // every buffer its kernels name; captured and instantiated on a miss.
 static int mixed_graph(Batch& B, int fmt, int interval, bool resident) {
     MixedWork* w = B.mixed;
-    const int key[GraphCache<MxArgs>::kKeys] = {fmt, interval, w->args.line, resident ? 1 : 0};
+    const int key[GraphCache<MxArgs>::kKeys] = {fmt, interval, w->args.line, resident ? 1 + w->res->absent : 0};
     w->exec = w->graphs.find(key, B.tiling_gen, w->args);
     if (w->exec) return EAFP_OK;
     EAFP_TRY(hipStreamSynchronize(B.stream));   // no earlier launch of a graph that make_room may drop
@@ -2164,7 +2164,10 @@ static int mixed_steps(Batch& B, const eafp_mixed_opts& o, int fmt, int interval
             counter_add(CTR_LAUNCHES, 1);
             EAFP_TRY(hipEventRecord(w->ev[launched & 1], B.stream));
             ++launched;
-            if (resident) w->res->tag += (unsigned)tags;
+            if (resident) {
+                w->res->tag += (unsigned)tags;
+                ++w->res->launches;
+            }
             if (resident && w->res->tag > 0xF0000000u - 2 * (unsigned)tags) {   // begin the tags again
                 EAFP_TRY(hipStreamSynchronize(B.stream));
                 if (finished() < 0) {
@@ -2206,11 +2209,13 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
     int aside = 0;
     // a step's tags have to fit the 32 bits several times over (resident.hpp);
     // longer steps, of millions of iterations, stream
-    if (B.resident_mixed && w->res && !w->res->given_up && resident_tags(*w->res, interval) < RES_STEP_TAGS) {
+    if (B.resident_mixed && w->res && w->res->usable() && resident_tags(*w->res, interval) < RES_STEP_TAGS) {
         const ResPlan& p = w->res->plan;
         const ResidentGate held(p.members);
+        const auto since = std::chrono::steady_clock::now();
         EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, MX_RESIDENT, &given_up, &aside));
-        w->res->given_up = given_up;
+        if (given_up) w->res->gave_up(since);
+        w->res->aside += aside;
     }
     if (given_up) EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, MX_STREAM, &given_up, &aside));
     else if (aside) EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, MX_SET_ASIDE, &given_up, &aside));
@@ -2254,11 +2259,12 @@ int time_resident_mixed(Batch& B, int fmt, int precond, int iters, float* ms) {
     EAFP_TRY_RC(check_mixed(B, o));
     EAFP_TRY_RC(ensure_mixed(B, fmt));
     MixedWork* w = B.mixed;
-    if (!w->res || w->res->given_up) return EAFP_OK;
+    if (!w->res || !w->res->usable()) return EAFP_OK;
     w->args.line = precond == EAFP_PRECOND_ZLINE ? 1 : 0;
     ResDevice& D = *w->res;
     EAFP_TRY_RC(rmx_prepare(fmt, w->args.line != 0, w->res_cq, D.plan.slots));
     const ResidentGate held(D.plan.members);
+    const auto since = std::chrono::steady_clock::now();
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
         EAFP_TRY_RC(mixed_start(B, o, fmt));
         EAFP_TRY_RC(D.arm(resident_tags(D, iters), B.stream));
@@ -2269,7 +2275,7 @@ int time_resident_mixed(Batch& B, int fmt, int precond, int iters, float* ms) {
         EAFP_TRY(hipStreamSynchronize(B.stream));
     }
     if (*w->host_cnt < 0) {
-        D.given_up = true;
+        D.gave_up(since);
         return EAFP_OK;
     }
     EAFP_TRY(hipEventElapsedTime(ms, w->t0, w->t1));
@@ -2314,5 +2320,7 @@ int time_mixed_kernels(Batch& B, int fmt, int precond, int reps, float* ms_spmv,
     if (ms_update) *ms_update = tot_u / (float)reps;
     return EAFP_OK;
 }
+
+ResDevice* resident_mixed(const Batch& B) { return B.mixed ? B.mixed->res.get() : nullptr; }
 
 }  // namespace eafp

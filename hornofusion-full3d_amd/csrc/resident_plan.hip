@@ -258,6 +258,13 @@ int ResDevice::create(ResPlan&& p, std::unique_ptr<ResDevice>& out, hipStream_t 
     return EAFP_OK;
 }
 
+constexpr int RES_RETRY = 100;
+void ResDevice::gave_up(std::chrono::steady_clock::time_point since) {
+    const auto now = std::chrono::steady_clock::now();
+    retry = now + RES_RETRY * (now - since);
+    ++given_up;
+}
+
 ResLaunch ResDevice::launch() const {
     ResLaunch L{};
     L.items = items.p;
@@ -268,7 +275,7 @@ ResLaunch ResDevice::launch() const {
     L.T = plan.T;
     L.slots = slots.p;
     L.gate = gate.p;
-    L.expected = plan.members;
+    L.expected = plan.members + absent;
     return L;
 }
 

@@ -1,6 +1,7 @@
 // resident_plan.hpp -- host side of the resident solvers: which batches
 // they take, the teams, and the launch's device tables.
 #pragma once
+#include <chrono>
 #include <memory>
 #include <vector>
 
@@ -67,7 +68,15 @@ struct ResDevice {
     DevBuf<u64> slots;
     DevBuf<unsigned> gate;
     unsigned tag = 1;             // first tag of the next launch
-    bool given_up = false;        // a launch did not get its CUs: stream from now on
+    // A launch that did not get its CUs has cost time (resident.hpp), and the
+    // batch streams until RES_RETRY times as long has passed: with the CUs held
+    // by others for good, a hundredth of the time is lost, and after a single
+    // collision the solves are on chip again.
+    std::chrono::steady_clock::time_point retry{};
+    bool usable() const { return std::chrono::steady_clock::now() >= retry; }
+    void gave_up(std::chrono::steady_clock::time_point since);
+    long long launches = 0, given_up = 0, aside = 0;   // of resident launches, given up, systems set aside
+    int absent = 0;               // work-groups that a launch waits for and that never come (tests)
     int init(ResPlan&& p, hipStream_t stream);
     ResLaunch launch() const;
     // `out` stays empty, and the batch streams, where the plan is not ok or the

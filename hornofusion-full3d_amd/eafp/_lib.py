@@ -32,7 +32,8 @@ EXPORTS = (
     "eafp_tdma_solve_batch", "eafp_batch_create", "eafp_batch_upload",
     "eafp_batch_solve_fp64", "eafp_batch_solve_mixed", "eafp_batch_download",
     "eafp_batch_info", "eafp_batch_set_tiling", "eafp_batch_set_columns", "eafp_batch_get_columns",
-    "eafp_batch_time_kernels", "eafp_batch_autotune", "eafp_batch_components", "eafp_batch_destroy",
+    "eafp_batch_time_kernels", "eafp_batch_autotune", "eafp_batch_components", "eafp_batch_resident", "eafp_batch_disturb",
+    "eafp_batch_destroy",
     "eafp_get_counters", "eafp_version",
 )
 
@@ -95,6 +96,16 @@ class Counters(ctypes.Structure):
     """eafp_counters: process-wide activity counters of the library."""
     _fields_ = [("uploads", ctypes.c_longlong), ("labelled", ctypes.c_longlong),
                 ("graph_captures", ctypes.c_longlong), ("graph_launches", ctypes.c_longlong)]
+
+
+class Resident(ctypes.Structure):
+    """eafp_resident: what a solver of a batch keeps on chip."""
+    _fields_ = [("work_groups", ctypes.c_int), ("teams", ctypes.c_int), ("team_size", ctypes.c_int),
+                ("in_use", ctypes.c_int), ("launches", ctypes.c_longlong), ("given_up", ctypes.c_longlong),
+                ("set_aside", ctypes.c_longlong)]
+
+
+DISTURB_ABSENT, DISTURB_TAG, DISTURB_PAUSE = 0, 1, 2
 
 
 class Stats(ctypes.Structure):
@@ -182,6 +193,10 @@ def load():
     L.eafp_batch_autotune.restype = i
     L.eafp_batch_components.argtypes = [vp, i, ip, ip]
     L.eafp_batch_components.restype = i
+    L.eafp_batch_resident.argtypes = [vp, i, ctypes.POINTER(Resident)]
+    L.eafp_batch_resident.restype = i
+    L.eafp_batch_disturb.argtypes = [vp, i, i, ctypes.c_uint]
+    L.eafp_batch_disturb.restype = i
     L.eafp_get_counters.argtypes = [ctypes.POINTER(Counters)]
     L.eafp_get_counters.restype = i
     L.eafp_batch_destroy.argtypes = [vp]

@@ -343,6 +343,16 @@ class Batch:
         check(self._L.eafp_batch_components(self._h, int(s), ctypes.byref(n), cells), "eafp_batch_components")
         return n.value, [cells[q] for q in range(n.value)] if n.value <= 4 else []
 
+    def resident(self, solver):
+        """What ``solver`` keeps on chip (eafp_batch_resident), as a dict."""
+        r = _lib.Resident()
+        check(self._L.eafp_batch_resident(self._h, solver, ctypes.byref(r)), "eafp_batch_resident")
+        return {n: getattr(r, n) for n, _ in r._fields_}
+
+    def disturb(self, solver, what, value=0):
+        """Brings about what is rare, for tests (eafp_batch_disturb)."""
+        check(self._L.eafp_batch_disturb(self._h, solver, what, value), "eafp_batch_disturb")
+
     def download(self, s, phi=None):
         nr, nth, nz = self.shapes[s]
         if phi is None:

@@ -373,6 +373,37 @@ int eafp_batch_autotune(eafp_batch* b, int solver, int coef_format, int reps, in
  * src/mod_pressure_3d.f90:261-265). */
 int eafp_batch_components(eafp_batch* b, int s, int* nsingular, int cells[4]);
 
+/* What a solver of the batch keeps on chip (solver as for
+ * eafp_batch_time_kernels; 1 and 2 have one form), for diagnostics and tests.
+ * All 0 before the solver's first solve, and where the batch has no such form.
+ * A launch that does not get its compute units in time (another process holds
+ * them) is given up, and that solve runs with the streaming kernels; so do the
+ * next ones until a hundred times the time lost has passed.  No reference
+ * counterpart. */
+typedef struct eafp_resident {
+    int work_groups;         /* of a launch; 0: no such form */
+    int teams;               /* the groups of them that hold a system each */
+    int team_size;           /* work-groups of a team; 0: teams of different sizes */
+    int in_use;              /* the next solve takes this form */
+    long long launches;
+    long long given_up;      /* launches that did not get their compute units */
+    long long set_aside;     /* systems that diverged and were solved again, streaming */
+} eafp_resident;
+
+int eafp_batch_resident(const eafp_batch* b, int solver, eafp_resident* out);
+
+/* Brings about, for tests, what is rare: launches from now on wait for `value`
+ * work-groups that never come and are given up (ABSENT; 0 ends it), the next
+ * launch's sums are numbered from `value` on, which is not below the present
+ * number (TAG; they begin again at 1 before 32 bits end), a solve within `value`
+ * seconds streams as if a launch had been given up before (PAUSE; 0 ends it).
+ * After the solver's first solve only (EAFP_ERR_STATE).  No reference
+ * counterpart. */
+#define EAFP_DISTURB_ABSENT 0
+#define EAFP_DISTURB_TAG 1
+#define EAFP_DISTURB_PAUSE 2
+int eafp_batch_disturb(eafp_batch* b, int solver, int what, unsigned value);
+
 int eafp_batch_destroy(eafp_batch* b);
 
 /* Process-wide activity counters, for diagnostics and tests: systems packed
