@@ -515,7 +515,7 @@ static int solve_fp64_resident(Batch& B, int max_iter, double tol, eafp_stats* s
     *done = 0;
     EAFP_TRY(hipEventRecord(w->t0, B.stream));
     EAFP_TRY_RC(start_resident64(B, D, w->slot1.p, w->cst.p, tol, max_iter, RES_ITERS));
-    const ResidentGate held(D.plan.members);
+    const ResidentGate held(D.plan.places());
     const auto since = std::chrono::steady_clock::now();
     for (bool first = true;; first = false) {
         EAFP_TRY_RC(launch_resident64(B, D, w->args, RES_ITERS, first));
@@ -604,7 +604,7 @@ int time_resident64(Batch& B, int iters, float* ms) {
     Cg64Work* w = B.cg64;
     if (!w->res || !w->res->usable()) return EAFP_OK;
     ResDevice& D = *w->res;
-    const ResidentGate held(D.plan.members);
+    const ResidentGate held(D.plan.places());
     const auto since = std::chrono::steady_clock::now();
     iters = std::min(iters, RES_ITERS);
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code

@@ -2211,7 +2211,7 @@ int solve_mixed(Batch& B, const eafp_mixed_opts& o, eafp_stats* stats) {
     // longer steps, of millions of iterations, stream
     if (B.resident_mixed && w->res && w->res->usable() && resident_tags(*w->res, interval) < RES_STEP_TAGS) {
         const ResPlan& p = w->res->plan;
-        const ResidentGate held(p.members);
+        const ResidentGate held(p.places());
         const auto since = std::chrono::steady_clock::now();
         EAFP_TRY_RC(mixed_steps(B, o, fmt, interval, MX_RESIDENT, &given_up, &aside));
         if (given_up) w->res->gave_up(since);
@@ -2263,7 +2263,7 @@ int time_resident_mixed(Batch& B, int fmt, int precond, int iters, float* ms) {
     w->args.line = precond == EAFP_PRECOND_ZLINE ? 1 : 0;
     ResDevice& D = *w->res;
     EAFP_TRY_RC(rmx_prepare(fmt, w->args.line != 0, w->res_cq, D.plan.slots));
-    const ResidentGate held(D.plan.members);
+    const ResidentGate held(D.plan.places());
     const auto since = std::chrono::steady_clock::now();
     for (int rep = 0; rep < 2; ++rep) {   // the first one settles caches and code
         EAFP_TRY_RC(mixed_start(B, o, fmt));

@@ -35,6 +35,9 @@ struct ResPlan {
     std::vector<int2> member;
     int nslot = 0;                            // slots of all teams
     long xlen = 0;                            // elements of the exchange buffer
+    // the CUs it takes: teams of one do not wait for each other, but others'
+    // launches would wait for them, longer than the gate does where lists are long
+    int places() const { return members > 0 ? members : nteam; }
 };
 
 // The plan for a batch, or !ok when a system fits no team.  `xpitch`: the

@@ -1,0 +1,22 @@
+"""Host-side check of the resident solvers' turns (CPU only): builds
+tests/resident_gate_check.cpp with the library's own gate and runs it."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC) and shutil.which("hipcc") is None, reason="hipcc not available")
+def test_turns(tmp_path):
+    exe = tmp_path / "resident_gate_check"
+    cmd = [HIPCC if os.path.exists(HIPCC) else "hipcc", "-x", "hip", "--offload-arch=gfx950",
+           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-O1", "-std=c++17",
+           "-o", str(exe), os.path.join(HERE, "resident_gate_check.cpp"), "-lpthread"]
+    subprocess.run(cmd, check=True, capture_output=True, timeout=300)
+    out = subprocess.run([str(exe)], capture_output=True, text=True, timeout=100)
+    assert out.returncode == 0, out.stdout + out.stderr
+    assert out.stdout.startswith("ok "), out.stdout
