@@ -61,7 +61,10 @@ struct SysGeom {
 // Lays out the systems' cells in one arena: fills nr/nth/nz/n/off and the
 // division reciprocals of every entry of g (whose nr, nth, nz are set) and
 // returns the arena length.  Every system starts at a 32-cell boundary, so
-// its FP64 arrays start 256-byte aligned.
+// its FP64 arrays start 256-byte aligned, and ROW_PAD cells or more behind the
+// one before: the resident mixed kernel reads the last row to the end of a
+// lane's cells, which are nobody's then.
+constexpr int ROW_PAD = 7;
 inline long layout_systems(std::vector<SysGeom>& g) {
     long off = 0;
     for (SysGeom& s : g) {
@@ -69,7 +72,7 @@ inline long layout_systems(std::vector<SysGeom>& g) {
         s.off = off;
         s.inv_nz = 1.0f / (float)s.nz;
         s.inv_nth = 1.0f / (float)s.nth;
-        off += (s.n + 31) / 32 * 32;
+        off += (s.n + ROW_PAD + 31) / 32 * 32;
     }
     return off;
 }
