@@ -59,6 +59,10 @@ class ResidentGate {
     int dev_, n_;
 };
 
+// Launches that the autotuner times of a resident form; it keeps the least time,
+// so that one launch held up does not send a batch to the streaming kernels.
+constexpr int RES_TIMED = 5;
+
 // A plan's tables on the device: some kilobytes, as rows are exchanged through an
 // array that the solver's resident kernel does not use otherwise, and given
 // back should the solver run out of memory later.

@@ -99,3 +99,25 @@ for n in with_it:
 
 def test_without_pinned_memory(tmp_path):
     limits.run(tmp_path, PINNED)
+
+
+SLOW = '''
+ps = systems.make_system(2, 0, (35, 66, 49))
+for solver in (eafp.Batch.SOLVER_FP64, eafp.Batch.SOLVER_MIXED_ZLINE):
+    with eafp.Batch.from_systems([ps]) as b:
+        shim.shim_slow(-1)
+        quiet = b.autotune(solver, _lib.COEF_BF16, reps=2)
+        calls = shim.shim_times()
+        shim.shim_slow(calls)        # the last launch that is timed
+        held_up = b.autotune(solver, _lib.COEF_BF16, reps=2)
+        assert shim.shim_times() == calls
+        shim.shim_slow(-1)
+        print("case slow", solver, calls, quiet, held_up, flush=True)
+        # the streaming kernels take twice as long on this mesh
+        assert held_up["ms_per_iter"] < 1.5 * quiet["ms_per_iter"]
+        assert b.resident(solver)["in_use"]
+'''
+
+
+def test_one_launch_held_up_does_not_decide(tmp_path):
+    limits.run(tmp_path, SLOW)
