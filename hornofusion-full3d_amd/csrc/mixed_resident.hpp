@@ -22,13 +22,13 @@
 // The arithmetic per cell is k_mspmv's and k_mupdate_line's; the order of the
 // sums differs.
 //
-// What bounds it: 604,800 cells on 128 work-groups take 8.7 us per BF16 z-line
-// iteration (17.5 streaming), 5.6 of it the two sums and the exchange of z;
-// eight such systems at once, 32 work-groups each, take 15.5 us (50
-// streaming), 8.6 of it the cells (the vector ALU: about 270 instructions per
-// quad), 6.5 the sums and the exchange.  4.8 million cells on 256 work-groups
-// take 20.5 us (60 streaming); its weights cross from the memory-side cache at
-// 10 TB/s in the stencil.
+// What bounds it: 604,800 cells on 256 work-groups take 8.4 us per BF16 z-line
+// iteration (17.5 streaming), the waves waiting 74 % of it for the two sums and
+// the exchange of z and the vector ALU busy 21 %; eight such systems at once,
+// 32 work-groups each, take 15.9 us (50 streaming), the vector ALU busy 55 % of
+// it (261 instructions per quad).  4.8 million cells on 256 work-groups take
+// 21.4 us (60 streaming), the vector ALU busy 36 %; 69 MB per iteration come
+// from beyond the L2s, 3.2 TB/s over the whole of it.
 #pragma once
 #include "mixed.hpp"
 #include "resident_plan.hpp"
@@ -41,8 +41,6 @@ struct RMxArgs {
     float* xz;           // exchange buffer, rows of nl*CQ quads
     int interval;
 };
-
-constexpr int RMX_MAX_NZ = 256;        // cells of the longest row a wave holds
 
 __host__ __device__ __forceinline__ int rmx_lanes(int nz, int cq) { return (nz + 4 * cq - 1) / (4 * cq); }
 __host__ __device__ constexpr size_t rmx_scratch() { return (sizeof(TeamLds) + 15) / 16 * 16; }

@@ -15,7 +15,7 @@
 // word, so a sum costs one store and one load through memory, and all
 // members add the same words in the same order: the same bits everywhere.
 // Measured on MI355X (store to the last member's sum): 1.1 us for 2..16
-// members, 1.9 us for 32, 3.0 us for 256.  The slots are double-buffered by
+// members, 1.9 us for 32, 2.5 us for 256.  The slots are double-buffered by
 // the tag's parity: a member stores sum n+2 only after sum n+1, which every
 // member joins after it has read sum n.
 //
@@ -34,6 +34,10 @@
 // Past the gate every wait ends because all the members run; should one
 // last WAIT_TICKS all the same, the work-group raises the same mark and
 // leaves.
+//
+// How long a sum takes also hangs on where the slots lie in memory: the same
+// code on the same mesh took 2.4 or 2.6 us per FP64 iteration of 18x36x24, and
+// 18.5 or 20.3 for 32 uneven systems, with the slots at other addresses.
 #pragma once
 #include <algorithm>
 
