@@ -1648,14 +1648,18 @@ __global__ __launch_bounds__(BLOCK) void k_mreplace_line(MxArgs a) {
 // begins again with the streaming kernels and ends where it always did: here it
 // is set aside (status MX_ASIDE, counted in ndone[1]), the others go on on
 // chip, and k_mrestart takes it up once they are done.  A
-// system counts as diverging when its residual is four times the first one or
-// 64 times the least so far: over 19286 solves of drawn systems, all 177 that did
-// not converge passed that (half of them within 20 steps of 2000, the last
-// after 396), and so did 25 of the 19109 that did converge, which then only take the longer
-// way.  A system of fewer than 512 cells is left
-// alone: the inner CG can solve it within a step, and its residual then jumps
-// up and down with either kernel before it gets there.
-constexpr double MX_FAR_FIRST = 4.0, MX_FAR_LEAST = 64.0;
+// system counts as diverging when its residual is MX_FAR_FIRST times the first
+// one or MX_FAR_LEAST times the least so far; at max_steps, the lower MX_END_*
+// times will do.  Over 21305 solves of drawn systems, 80 of them of 120x240x168,
+// all 220 that did not converge passed 16 or 1024 (half of them within 26 steps
+// of 2000, on average after 90), and so did one of the 21085 that did.  With 4 and
+// 64 it is 11 and 41 steps, but 45 systems that converge begin again all the same,
+// a fifth of those of 120x240x168 with BF16 weights and the z-line preconditioner
+// among them: such a solve takes 265 ms instead of 105.  A system of fewer than
+// 512 cells is left alone: the inner CG can solve it within a step, and its
+// residual then jumps up and down with either kernel before it gets there.
+constexpr double MX_FAR_FIRST = 16.0, MX_FAR_LEAST = 1024.0;
+constexpr double MX_END_FIRST = 4.0, MX_END_LEAST = 64.0;
 constexpr int MX_FAR_CELLS = 512;
 constexpr int MX_ASIDE = -1;   // MxStat::status, between k_mcount and k_mrestart only
 __global__ __launch_bounds__(BLOCK) void k_mcount(MxArgs a, unsigned* gate, unsigned tags) {
@@ -1665,7 +1669,9 @@ __global__ __launch_bounds__(BLOCK) void k_mcount(MxArgs a, unsigned* gate, unsi
         // all loads first: one after another they cost the step a microsecond
         MxStat& S = a.stat[1][s];
         const int status = S.status, cells = a.geom[s].n;
-        const double now = S.res_l2, far = fmin(MX_FAR_FIRST * S.res_first, MX_FAR_LEAST * S.res_least);
+        const bool end = status == EAFP_STOP_MAX_ITER;
+        const double now = S.res_l2, far = fmin((end ? MX_END_FIRST : MX_FAR_FIRST) * S.res_first,
+                                                (end ? MX_END_LEAST : MX_FAR_LEAST) * S.res_least);
         int done = S.done;
         bool aside = status == MX_ASIDE;
         if ((gate != nullptr) & !aside & (status != EAFP_STOP_CONVERGED) & (cells >= MX_FAR_CELLS) & (now > far)) {

@@ -24,7 +24,7 @@
 //
 // What bounds it: 604,800 cells on 256 work-groups take 8.4 us per BF16 z-line
 // iteration (17.5 streaming), the waves waiting 74 % of it for the two sums and
-// the exchange of z and the vector ALU busy 21 %; eight such systems at once,
+// the exchange of z and the vector ALU busy 22 %; eight such systems at once,
 // 32 work-groups each, take 15.9 us (50 streaming), the vector ALU busy 55 % of
 // it (261 instructions per quad).  4.8 million cells on 256 work-groups take
 // 21.4 us (60 streaming), the vector ALU busy 36 %; 69 MB per iteration come

@@ -51,3 +51,21 @@ def test_only_the_diverging_systems_begin_again(precond, place):
             assert np.array_equal(phi[q], phi_w[q]) and st[q]["n_iter"] == st_w[q]["n_iter"]
     # the others' steps on chip, one launch each, then every step of the two
     assert launches >= max(st[q]["n_refine"] for q in range(5) if q not in bad) + 120
+
+
+# systems that converge after their residual was up to 373 times its least
+UNSTEADY = [((71, 15, 86), 297172762, _lib.COEF_FP32, _lib.PRECOND_ZLINE),
+            ((11, 78, 71), 1045996112, _lib.COEF_FP32, _lib.PRECOND_JACOBI),
+            ((13, 36, 47), 824138931, _lib.COEF_BF16, _lib.PRECOND_JACOBI),
+            ((15, 24, 23), 172062608, _lib.COEF_BF16, _lib.PRECOND_ZLINE)]
+
+
+@pytest.mark.parametrize("shape,seed,fmt,precond", UNSTEADY)
+def test_an_unsteady_system_stays_on_chip(shape, seed, fmt, precond):
+    print(f"case unsteady {shape} fmt {fmt} precond {precond}", flush=True)
+    with eafp.Batch.from_systems([systems.make_system(4, 257 * seed, shape)]) as b:
+        c0 = eafp.counters()["graph_launches"]
+        st = b.solve_mixed(tol=1e-10, coef_format=fmt, precond=precond)[0]
+        launches = eafp.counters()["graph_launches"] - c0
+    assert st["status"] == "converged"
+    assert launches <= st["n_refine"] + 2       # one per refinement step: nothing solved again
