@@ -371,6 +371,7 @@ static int init_cg64(Batch& B, Cg64Work* w) {
         EAFP_TRY(hipMemset(w->p0.p, 0, n * sizeof(double)));
         EAFP_TRY(hipMemset(w->p1.p, 0, n * sizeof(double)));
         ResPlan plan = plan_resident64(B);
+        plan.ok = plan.ok && plan.xlen <= B.ncells;   // the rows cross through q
         EAFP_TRY_RC(ResDevice::create(std::move(plan), w->res, B.stream));
         if (w->res && !(pinned_alloc(&w->slots_host, B.nsys) && pinned_alloc(&w->gate_host, 1)))
             w->res.reset();   // nowhere to report to: the streaming kernels

@@ -1,6 +1,8 @@
 // Who may launch (ResidentGate in csrc/resident_plan.hip): threads with plans of
 // their own never hold more than the chip between them, come in the order in
-// which they asked, and a plan of teams of one takes places too.
+// which they asked, and a plan of teams of one takes places too.  And where the
+// rows cross: one double per cell for FP64, two floats for the mixed solver with
+// rows of four cells or more, no two systems in the same place.
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -54,7 +56,37 @@ static void hold(int n) {
     g_held.fetch_sub(n);
 }
 
+static int pitch1(int nz) { return (nz + 3) / 4 * 4; }
+static int pitch2(int nz) { return (nz + 7) / 8 * 8; }
+
+static void exchange() {
+    std::mt19937 rng(11);
+    for (int rep = 0; rep < 200; ++rep) {
+        std::vector<SysGeom> g(1 + rng() % 40);
+        for (auto& s : g) {
+            s = SysGeom{};
+            s.nr = 1 + (int)(rng() % 30);
+            s.nth = 1 + (int)(rng() % 40);
+            s.nz = (rep % 2 ? 4 : 1) + (int)(rng() % 60);
+        }
+        const long ncells = layout_systems(g);
+        for (int (*pt)(int) : {pitch, pitch1, pitch2}) {
+            const ResPlan p = plan_resident(g, kLim, pt);
+            if (!p.ok) continue;
+            if (pt == pitch) CHECK(p.xlen <= ncells, "%ld of %ld", p.xlen, ncells);
+            if (rep % 2) CHECK(p.xlen <= 2 * ncells, "%ld of %ld", p.xlen, 2 * ncells);
+            std::vector<std::pair<long, long>> part;
+            for (const ResItem& I : p.items) part.push_back({I.xoff, I.xoff + (long)I.nr * I.nth * pt(I.nz)});
+            std::sort(part.begin(), part.end());
+            CHECK(part.front().first == 0 && part.back().second <= p.xlen, "ends");
+            for (size_t q = 1; q < part.size(); ++q)
+                CHECK(part[q].first >= part[q - 1].second && part[q].first % 32 == 0, "part %zu", q);
+        }
+    }
+}
+
 int main() {
+    exchange();
     // plans and what they take
     const ResPlan many = plan(5000, 8, 8, 8), one = plan(1, 60, 120, 84), few = plan(3, 20, 30, 33);
     CHECK(many.ok && many.T == 1 && many.members == 0, "teams of %d", many.T);

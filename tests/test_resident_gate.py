@@ -1,4 +1,5 @@
-"""Host-side check of the resident solvers' turns (CPU only): builds
+"""Host-side check of the resident solvers' turns and of the places through
+which they exchange rows (CPU only): builds
 tests/resident_gate_check.cpp with the library's own gate and runs it."""
 import os
 import shutil
